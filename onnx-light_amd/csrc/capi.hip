@@ -1146,7 +1146,7 @@ int QLinearConv(const onnxl_amd_tensor *x, const onnxl_amd_tensor *x_scale, cons
   const bool implicit = gemm && ConvImplicit(g, *y);  // the GEMM epilogue requantizes
   const size_t col_bytes = implicit ? ConvImplicitScratch(g) : (gemm ? ConvColBytes(g) : 0);
   const size_t acc_off = Scratch::Round(col_bytes);
-  const size_t acc_bytes = gemm && !implicit ? (size_t)(g.N * g.M * g.P) * 4 : 0;
+  const size_t acc_bytes = gemm && g.G > 1 ? (size_t)(g.N * g.M * g.P) * 4 : 0;
   Staging st(stream, acc_off + acc_bytes, {x, w, w_scale, w_per_channel ? w_zp : nullptr, has_bias ? bias : nullptr},
              {y});
   const uint8_t *xd = static_cast<const uint8_t *>(st.In(x));
@@ -1171,8 +1171,8 @@ int QLinearConv(const onnxl_amd_tensor *x, const onnxl_amd_tensor *x_scale, cons
         col = static_cast<uint8_t *>(st.Extra());
         LaunchImToCol(g, xd, (uint8_t)xz, static_cast<uint8_t *>(st.Extra()), stream);
       }
-      // group 1 on the pipelined kernel: the GEMM epilogue requantizes each
-      // output channel's row itself; otherwise int32 sums, then the pass
+      // group 1: the GEMM epilogue requantizes each output channel's row
+      // itself; otherwise int32 sums, then the pass
       IGemmParams p = implicit ? ConvImplicitGemm(g, xd, x->data_type == kUint8, xz, wd, w->data_type == kUint8, wzd,
                                                   wz, yd, st.Extra(), stream)
                                : ConvGemmParams(g, wd, w->data_type == kUint8, wzd, wz, col, x->data_type == kUint8,
@@ -1187,7 +1187,7 @@ int QLinearConv(const onnxl_amd_tensor *x, const onnxl_amd_tensor *x_scale, cons
       p.row_xs = q.x_scale;
       p.row_ys = q.y_scale;
       p.row_bias = q.bias;
-      if (implicit || (g.G == 1 && IGemmFastEligible(p))) {
+      if (implicit || g.G == 1) {
         LaunchIGemm(p, stream);
       } else {
         LaunchConvGemm(g, wd, w->data_type == kUint8, wzd, wz, col, x->data_type == kUint8, xz, acc, stream);

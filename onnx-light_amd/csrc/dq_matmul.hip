@@ -6,7 +6,9 @@
 //  - float8e4m3fn weights, FLOAT scales per column or per tensor, Cast to
 //    BFLOAT16, bf16 activations (prefill): the pipelined MFMA core with the
 //    weight decoded exactly to bf16 as it is read from LDS and the scale
-//    applied to the fp32 sums (mfma_gemm.hpp, kBf16F8).
+//    applied to the fp32 sums (mfma_gemm.hpp, kBf16F8); the small-tile GEMM
+//    for few outputs, and for the shapes and alignments the core does not
+//    take, there with each weight rounded as the chain rounds it.
 //  - anything else the C ABI accepts: the weight is dequantised into scratch
 //    with the chain's exact rounding, then multiplied by the 16-bit MatMul.
 #include <algorithm>
@@ -15,6 +17,7 @@
 #include "device_codecs.hpp"
 #include "kernels.hpp"
 #include "mfma_gemm.hpp"
+#include "tile_gemm.hpp"
 
 namespace onnxl_amd {
 
@@ -24,31 +27,11 @@ void LaunchGemvQ4Tiled(const DqMatMulParams &p, hipStream_t stream);
 size_t GemvQ4ScratchBytes(const DqMatMulParams &p);
 size_t GemvQ4Counters(const DqMatMulParams &p);
 void LaunchGemvQ4(const DqMatMulParams &p, void *scratch, unsigned *counters, hipStream_t stream);
+void LaunchHTile(const mg::GemmArgs &g, bool bf16, bool big, hipStream_t s);
+void LaunchHTileBT(const mg::GemmArgs &g, bool bf16, bool big, hipStream_t s);
+void LaunchF8Tile(const mg::GemmArgs &g, bool chain, bool big, hipStream_t s);
 
 namespace {
-
-// ---------------------------------------------------------------------------
-// Generic 16-bit MatMul for shapes the MFMA core does not take: one thread per
-// output, fp32 accumulation in k order.  TB: B given transposed, [N, K].
-template <bool BF16, bool TB = false>
-__global__ __launch_bounds__(256) void HMatMulSimpleKernel(const HMatMulParams p) {
-  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t m = blockIdx.y;
-  const int64_t b = blockIdx.z;
-  if (n >= p.N) return;
-  int64_t ao, bo;
-  BatchOffsets(p.bm, b, ao, bo);
-  const uint16_t *a = p.A + ao + m * p.K;
-  const uint16_t *w = p.B + bo + (TB ? n * p.K : n);
-  const int64_t wstep = TB ? 1 : p.N;
-  float acc = 0.f;
-  for (int64_t k = 0; k < p.K; ++k) {
-    const float x = BF16 ? Bf16ToF32(a[k]) : F16ToF32(a[k]);
-    const float y = BF16 ? Bf16ToF32(w[k * wstep]) : F16ToF32(w[k * wstep]);
-    acc += x * y;
-  }
-  p.Y[(b * p.M + m) * p.N + n] = BF16 ? F32ToBf16(acc) : F32ToF16(acc);
-}
 
 mg::GemmArgs HArgs(const HMatMulParams &p) {
   mg::GemmArgs g{};
@@ -187,31 +170,22 @@ mg::GemmArgs Fp8Args(const DqMatMulParams &p) {
 void LaunchHMatMul(const HMatMulParams &p, hipStream_t stream) {
   if (p.M == 0 || p.N == 0 || p.batch == 0) return;
   const mg::GemmArgs g = HArgs(p);
-  if (mg::Eligible<mg::kH16>(g)) {
-    if (p.bf16) mg::Launch<mg::kH16, mg::kOutBf16, false, false, false>(g, stream);
-    else mg::Launch<mg::kH16, mg::kOutF16, false, false, false>(g, stream);
-    return;
-  }
-  const dim3 grid((unsigned)((p.N + 255) / 256), (unsigned)p.M, (unsigned)p.batch);
-  if (p.bf16) hipLaunchKernelGGL(HMatMulSimpleKernel<true>, grid, dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL(HMatMulSimpleKernel<false>, grid, dim3(256), 0, stream, p);
+  const bool small = tg::PrefersSmallTile(g);
+  if (small || !mg::Eligible<mg::kH16>(g)) LaunchHTile(g, p.bf16, !small, stream);
+  else if (p.bf16) mg::Launch<mg::kH16, mg::kOutBf16, false, false, false>(g, stream);
+  else mg::Launch<mg::kH16, mg::kOutF16, false, false, false>(g, stream);
 }
 
-// Y = A @ B^T for B given as [N, K] (batch 1): the MFMA core reading B's rows
-// like A's, else the simple kernel.
+// Y = A @ B^T for B given as [N, K] (batch 1).
 void LaunchHMatMulBT(const HMatMulParams &p, hipStream_t stream) {
   if (p.M == 0 || p.N == 0) return;
   const mg::GemmArgs g = HArgs(p);
-  if (p.batch == 1 && mg::EligibleBT(g)) {
-    if (p.bf16) mg::LaunchBT<mg::kOutBf16>(g, stream);
-    else mg::LaunchBT<mg::kOutF16>(g, stream);
-    return;
-  }
-  if (p.M > 65535 || p.batch > 65535) throw Unsupported("MatMul with B given as [N, K]: the one-thread-per-output "
-                                                       "kernel for N % 16 != 0 takes at most 65535 rows");
-  const dim3 grid((unsigned)((p.N + 255) / 256), (unsigned)p.M, (unsigned)p.batch);
-  if (p.bf16) hipLaunchKernelGGL((HMatMulSimpleKernel<true, true>), grid, dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL((HMatMulSimpleKernel<false, true>), grid, dim3(256), 0, stream, p);
+  if (p.N % 16 != 0 && p.M > 65535)
+    throw Unsupported("MatMul with B given as [N, K]: N % 16 != 0 takes at most 65535 rows");
+  const bool small = tg::PrefersSmallTile(g);
+  if (small || !mg::EligibleBT(g)) LaunchHTileBT(g, p.bf16, !small, stream);
+  else if (p.bf16) mg::LaunchBT<mg::kOutBf16>(g, stream);
+  else mg::LaunchBT<mg::kOutF16>(g, stream);
 }
 
 size_t DqMatMulScratchBytes(const DqMatMulParams &p) {
@@ -239,10 +213,10 @@ bool LaunchDqMatMul(const DqMatMulParams &p, void *scratch, size_t scratch_bytes
   }
   if (Fp8Eligible(p)) {
     const mg::GemmArgs g = Fp8Args(p);
-    if (mg::Eligible<mg::kBf16F8>(g)) {
-      LaunchFp8Gemm(g, stream);
-      return true;
-    }
+    const bool core = mg::Eligible<mg::kBf16F8>(g), small = tg::PrefersSmallTile(g);
+    if (core && !small) LaunchFp8Gemm(g, stream);
+    else LaunchF8Tile(g, /*chain=*/!core, !small, stream);
+    return true;
   }
   // general path: dequantise into scratch, then the 16-bit MatMul (K == 0
   // leaves nothing to dequantise and the MatMul writes zeros)

@@ -127,7 +127,7 @@ struct IGemmParams {
   // Device-resident scalars replacing alpha_scalar, beta_scalar, cs and zy
   // (kEpiInt32 / kEpiQuant8); need_cb / need_ra are set when za / zb is one.
   QDevScalars dev;
-  // kEpiQuant8Row (pipelined kernel only): row r uses the scale
+  // kEpiQuant8Row: row r uses the scale
   // row_xs * row_wscale[r or 0] / row_ys and adds row_bias[r] (if not null)
   // to the int32 sum exactly before the conversion.
   const float *row_wscale;
@@ -145,9 +145,6 @@ void LaunchIGemm(const IGemmParams &p, hipStream_t stream);
 // M, N, K, batch, bm, a_u8, b_u8, cs, zy, qmin, qmax, y_signed, dev and the
 // zero points za, zb given here (replaced by dev.za / dev.zb when set).
 void LaunchQlmExact(const IGemmParams &p, int32_t za, int32_t zb, hipStream_t stream);
-// Whether LaunchIGemm takes the pipelined MFMA kernel for p (kEpiQuant8Row
-// requires it).
-bool IGemmFastEligible(const IGemmParams &p);
 
 // ---------------------------------------------------------------------------
 // DequantizePacked, 32-value GGUF formats (ggml type codes 2, 3, 6, 7, 8, 9,

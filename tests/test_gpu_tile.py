@@ -1,0 +1,92 @@
+"""The small-tile GEMM (csrc/tile_gemm.hpp) at the edges of its 64 x 64 and
+128 x 128 tiles, its K steps and its guarded last step: rows that end inside a
+16-byte piece, matrices of less than one piece, one past and one short of a
+tile.  Integers against the oracle, bit for bit.  The 16-bit kinds use small
+integers times powers of two, whose fp32 sums are exact in any order, so the
+result is the exact sum rounded once to the output type."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1, 1), (2, 15, 3), (3, 130, 1), (1, 17, 7), (64, 128, 64), (65, 127, 63), (63, 129, 65), (5, 64, 16),
+          (129, 200, 130), (200, 1, 77), (31, 256, 15), (7, 2049, 9),
+          (1100, 72, 2100), (1025, 131, 2053)]  # more than 512 small tiles: 128 x 128 ones
+
+
+@pytest.fixture(scope="module")
+def dev(olamd):
+    olamd.init(0)
+    return torch.device("cuda:0")
+
+
+def _T(x, dev):
+    return torch.from_numpy(np.ascontiguousarray(x)).to(dev)
+
+
+def _offset(t):
+    """t at an address that is no multiple of 16 bytes (of its element size only)."""
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    buf[1:].copy_(t.reshape(-1))
+    return buf[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+@pytest.mark.parametrize("dts", [(np.uint8, np.int8), (np.int8, np.uint8)], ids=["u8s8", "s8u8"])
+def test_int8(olamd, oracle, dev, shape, dts):
+    M, K, N = shape
+    rng = np.random.default_rng(M * 7919 + K * 31 + N)
+    a = rng.integers(np.iinfo(dts[0]).min, np.iinfo(dts[0]).max + 1, (M, K)).astype(dts[0])
+    b = rng.integers(np.iinfo(dts[1]).min, np.iinfo(dts[1]).max + 1, (K, N)).astype(dts[1])
+    za = rng.integers(np.iinfo(dts[0]).min, np.iinfo(dts[0]).max + 1, M).astype(dts[0])
+    zb = rng.integers(np.iinfo(dts[1]).min, np.iinfo(dts[1]).max + 1, N).astype(dts[1])
+    ta, tb = _offset(_T(a, dev)), _offset(_T(b, dev))
+    y = olamd.matmul_integer(ta, tb, _T(za, dev), _T(zb, dev))
+    sums = (a.astype(np.int64) - za[:, None]) @ (b.astype(np.int64) - zb)
+    if M * K * N < 2_000_000:
+        assert np.array_equal(oracle.matmul_integer(a, b, za.tolist(), zb.tolist()), sums)
+    assert np.array_equal(y.cpu().numpy(), sums)
+    s = [np.array(v, np.float32) for v in (0.02, 0.004, 0.3)]
+    yz = np.array(3, dts[0])
+    q = olamd.qlinear_matmul(ta, s[0], np.array(za[0]), tb, s[1], np.array(zb[0]), s[2], yz)
+    if M * K * N < 2_000_000:
+        want = oracle.qlinear_matmul(a, s[0], int(za[0]), b, s[1], int(zb[0]), s[2], yz)
+    else:
+        sums = (a.astype(np.int64) - int(za[0])) @ (b.astype(np.int64) - int(zb[0]))
+        cs = np.float32(np.float32(s[0] * s[1]) / s[2])
+        info = np.iinfo(dts[0])
+        want = np.clip(np.rint(sums.astype(np.float32) * cs) + np.float32(yz), info.min, info.max).astype(dts[0])
+    assert np.array_equal(q.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_16_bit(olamd, dev, shape):
+    M, K, N = shape
+    g = torch.Generator(device=dev).manual_seed(K)
+    ints = lambda lo, hi, sh: torch.randint(lo, hi, sh, generator=g, device=dev, dtype=torch.int32)  # noqa: E731
+    a, b = ints(-2, 3, (2, M, K)), ints(-8, 9, (2, K, N))
+    exact = torch.stack([x.double() @ y.double() for x, y in zip(a, b)])
+    assert float(torch.stack([x.double().abs() @ y.double().abs() for x, y in zip(a, b)]).max()) < 2 ** 24
+    for dt in (torch.float16, torch.bfloat16):
+        y = olamd.matmul(_offset(a.to(dt)), _offset(b.to(dt)))
+        assert torch.equal(y, exact.to(torch.float32).to(dt)), dt
+    # fp8 weights under bf16 activations: codes that are small integers, power-of-two scales
+    scale = torch.pow(2.0, -ints(0, 4, (N,)).float())
+    w = b[0].to(torch.float8_e4m3fn)
+    y = olamd.dequantize_linear_matmul(a[0].to(torch.bfloat16), w, scale if N > 1 else scale.reshape(()), None, 1,
+                                       olamd.BFLOAT16)
+    assert torch.equal(y, (exact[0] * scale.double()).to(torch.float32).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 1, 64), (65, 63, 32), (130, 129, 320), (1100, 2101, 96)])
+def test_b_transposed(olamd, dev, M, N, K):
+    """The packed-weight product past the GEMVs: its decoded weight is [N, K]."""
+    g = torch.Generator(device=dev).manual_seed(N)
+    a = torch.randint(-2, 3, (M, K), generator=g, device=dev, dtype=torch.int32)
+    q = torch.randint(-8, 9, (N * K // 32, 32), generator=g, device=dev, dtype=torch.int32)
+    d = torch.full((N * K // 32, 1), 0.5, dtype=torch.float16, device=dev)
+    x = torch.cat((d.view(torch.uint8).view(-1, 2), q.to(torch.int8).view(torch.uint8)), dim=1).reshape(-1)
+    y = olamd.dequantize_packed_matmul(a.to(torch.float16), x, "gguf:q8_0", (N, K))
+    exact = a.double() @ (q.double().view(N, K) * 0.5).t().contiguous()
+    assert torch.equal(y, exact.to(torch.float32).to(torch.float16))
