@@ -83,7 +83,7 @@ constexpr int kStoreThrough = 16;
 //  kI8:     int8 / uint8 x int8 / uint8 -> int32 (v_mfma_i32_32x32x32_i8)
 //  kBf16F8: bf16 A x float8e4m3fn B with a per-column (or single) fp32 scale;
 //           B values enter the MFMA exactly (every e4m3fn value is a bf16
-//           value: the high half of its fp32 decode) and the column's scale
+//           value) and the column's scale
 //           multiplies the fp32 sum in the epilogue, Y = s_n * sum_k a q.
 //           The DequantizeLinear(FLOAT) -> Cast(BFLOAT16) chain instead rounds
 //           each s_n * q to bf16 first; the two differ by at most half a bf16
@@ -133,14 +133,15 @@ __device__ __forceinline__ unsigned PackBf16(float lo, float hi) {
   return r;
 }
 
-// Two floats that are bf16 values (fp8 decodes) -> packed bf16 pair, lo in
-// bits 0-15: their high halves, exact for such values.  Inline asm: the
-// compiler folds __builtin_amdgcn_perm of the two halves of one register pair
-// into a perm of the low half with itself.
-__device__ __forceinline__ unsigned HighHalves(v2f f) {
-  unsigned r;
-  asm("v_perm_b32 %0, %1, %2, %3" : "=v"(r) : "v"(f.y), "v"(f.x), "s"(0x07060302u));
-  return r;
+// Two float8e4m3fn codes (the low or the high pair of `x`) -> packed bf16
+// pair, exact: gfx950's scaled conversion with scale 1.  One instruction for
+// two weights, where an fp32 pair decode and a byte permute of its high halves
+// took two: bf16[4096,4096] x fp8[4096,14336] 368 -> 357 us.
+__device__ __forceinline__ int Fp8PairLo(int x) {
+  return __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x, 1.f, false));
+}
+__device__ __forceinline__ int Fp8PairHi(int x) {
+  return __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x, 1.f, true));
 }
 
 // One direct load: lane i's 16 bytes at `voffset` land at LDS address
@@ -545,12 +546,8 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
       if constexpr (KIND == kI8 && BU8) {
         rb[rbuf][j] ^= bflip;
       } else if constexpr (KIND == kBf16F8) {
-        // exact fp8 -> bf16: the high halves of the fp32 decode
-        const v2f f0 = __builtin_amdgcn_cvt_pk_f32_fp8(rb[rbuf][j].x, false);
-        const v2f f1 = __builtin_amdgcn_cvt_pk_f32_fp8(rb[rbuf][j].x, true);
-        const v2f f2 = __builtin_amdgcn_cvt_pk_f32_fp8(rb[rbuf][j].y, false);
-        const v2f f3 = __builtin_amdgcn_cvt_pk_f32_fp8(rb[rbuf][j].y, true);
-        bop[bbuf][j] = v4i{(int)HighHalves(f0), (int)HighHalves(f1), (int)HighHalves(f2), (int)HighHalves(f3)};
+        const int x = rb[rbuf][j].x, y = rb[rbuf][j].y;
+        bop[bbuf][j] = v4i{Fp8PairLo(x), Fp8PairHi(x), Fp8PairLo(y), Fp8PairHi(y)};
       }
     }
   };
@@ -600,7 +597,7 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
   // Instruction order inside a sub-step, pinned because the scheduler would
   // otherwise sink each LDS read next to its first use.
   constexpr int kReads = 4 + WB * (KIND == kBf16F8 ? 1 : 2);
-  constexpr int kDecodeValu = KIND == kBf16F8 ? 8 * WB : (KIND == kI8 ? (AU8 ? 16 : 0) + (BU8 ? 4 * WB : 0) + (CB ? 4 * WB : 0) : 0);
+  constexpr int kDecodeValu = KIND == kBf16F8 ? 4 * WB : (KIND == kI8 ? (AU8 ? 16 : 0) + (BU8 ? 4 * WB : 0) + (CB ? 4 * WB : 0) : 0);
   // A plain sub-step with `nvm` direct loads: each MFMA is preceded by its
   // share of the LDS reads two sub-steps ahead and followed by a direct load
   // and its share of the decode.  Reads issued all at once at the top of a

@@ -213,17 +213,16 @@ __global__ __launch_bounds__(256, 2) void TileGemmKernel(const GemmArgs p) {
       if constexpr (F8) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          // fp8 -> fp32 exactly; its high half is the bf16 value
           const int x = b[q][2 * h], y = b[q][2 * h + 1];
-          const v2f f0 = __builtin_amdgcn_cvt_pk_f32_fp8(x, false), f1 = __builtin_amdgcn_cvt_pk_f32_fp8(x, true);
-          const v2f f2 = __builtin_amdgcn_cvt_pk_f32_fp8(y, false), f3 = __builtin_amdgcn_cvt_pk_f32_fp8(y, true);
           v4i w;
           if constexpr (SRC == kSrcF8Chain) {
+            const v2f f0 = __builtin_amdgcn_cvt_pk_f32_fp8(x, false), f1 = __builtin_amdgcn_cvt_pk_f32_fp8(x, true);
+            const v2f f2 = __builtin_amdgcn_cvt_pk_f32_fp8(y, false), f3 = __builtin_amdgcn_cvt_pk_f32_fp8(y, true);
             const float *s = wsc[q] + 8 * h;
             w = v4i{(int)mg::PackBf16(f0.x * s[0], f0.y * s[1]), (int)mg::PackBf16(f1.x * s[2], f1.y * s[3]),
                     (int)mg::PackBf16(f2.x * s[4], f2.y * s[5]), (int)mg::PackBf16(f3.x * s[6], f3.y * s[7])};
           } else {
-            w = v4i{(int)mg::HighHalves(f0), (int)mg::HighHalves(f1), (int)mg::HighHalves(f2), (int)mg::HighHalves(f3)};
+            w = v4i{mg::Fp8PairLo(x), mg::Fp8PairHi(x), mg::Fp8PairLo(y), mg::Fp8PairHi(y)};
           }
           *reinterpret_cast<v4i *>(sb + wb[q] + 16 * h) = w;
         }
