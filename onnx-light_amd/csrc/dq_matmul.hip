@@ -6,8 +6,8 @@
 //  - float8e4m3fn weights, FLOAT scales per column or per tensor, Cast to
 //    BFLOAT16, bf16 activations (prefill): the pipelined MFMA core with the
 //    weight decoded exactly to bf16 as it is read from LDS and the scale
-//    applied to the fp32 sums (mfma_gemm.hpp, kBf16F8); the small-tile GEMM
-//    for few outputs, and for the shapes and alignments the core does not
+//    applied to the fp32 sums (mfma_gemm.hpp, kBf16F8); the decode GEMM
+//    (skinny_gemm.hpp) for a few rows; the small-tile GEMM for few outputs, and for the shapes and alignments the core does not
 //    take, there with each weight rounded as the chain rounds it.
 //  - anything else the C ABI accepts: the weight is dequantised into scratch
 //    with the chain's exact rounding, then multiplied by the 16-bit MatMul.
@@ -17,6 +17,7 @@
 #include "device_codecs.hpp"
 #include "kernels.hpp"
 #include "mfma_gemm.hpp"
+#include "skinny_gemm.hpp"
 #include "tile_gemm.hpp"
 
 namespace onnxl_amd {
@@ -29,6 +30,7 @@ size_t GemvQ4Counters(const DqMatMulParams &p);
 void LaunchGemvQ4(const DqMatMulParams &p, void *scratch, unsigned *counters, hipStream_t stream);
 void LaunchHTile(const mg::GemmArgs &g, bool bf16, bool big, hipStream_t s);
 void LaunchHTileBT(const mg::GemmArgs &g, bool bf16, bool big, hipStream_t s);
+void LaunchF8Skinny(const mg::GemmArgs &g, hipStream_t s);
 void LaunchF8Tile(const mg::GemmArgs &g, bool chain, bool big, hipStream_t s);
 
 namespace {
@@ -214,7 +216,8 @@ bool LaunchDqMatMul(const DqMatMulParams &p, void *scratch, size_t scratch_bytes
   if (Fp8Eligible(p)) {
     const mg::GemmArgs g = Fp8Args(p);
     const bool core = mg::Eligible<mg::kBf16F8>(g), small = tg::PrefersSmallTile(g);
-    if (core && !small) LaunchFp8Gemm(g, stream);
+    if (core && sk::PrefersSkinny(g, false, false)) LaunchF8Skinny(g, stream);
+    else if (core && !small) LaunchFp8Gemm(g, stream);
     else LaunchF8Tile(g, /*chain=*/!core, !small, stream);
     return true;
   }

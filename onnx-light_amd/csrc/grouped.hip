@@ -19,6 +19,8 @@
 //     once.  Shapes the core does not take (K % 32 != 0, N % 16 != 0,
 //     unaligned payloads) run GroupedSimpleKernel, one thread per output
 //     element summing in order over k.
+// fp8 experts with few pairs each take the decode GEMM (skinny_gemm.hpp)
+// instead, one launch without the routing pass.
 // The sums are fp32 over exact products of 16-bit values, as the reference's
 // (km/kernel_grouped_matmul.cc:22-46); with a bias, the sum is rounded to the
 // output dtype, the bias added in fp32 and the result rounded again.
@@ -26,8 +28,12 @@
 #include "device_codecs.hpp"
 #include "kernels.hpp"
 #include "mfma_gemm.hpp"
+#include "skinny_gemm.hpp"
 
 namespace onnxl_amd {
+
+void LaunchF8SkinnyGrouped(const mg::GemmArgs &g, const void *idx, int idx64, hipStream_t s);
+
 namespace {
 
 constexpr int kRouteThreads = 1024;
@@ -255,12 +261,6 @@ void LaunchDqGroupedMatMul(const DqGroupedParams &p, hipStream_t stream) {
     LaunchGroupedMatMul(g, stream);
     return;
   }
-  // 256 x 256 tiles (as configuration 4's fp8 GEMM) when K takes whole K
-  // steps; the routing then counts 256-column tiles
-  GroupedParams gp = p.g;
-  const bool wide = p.g.K % 64 == 0;
-  if (wide) gp.nbn = (p.g.N + 255) / 256;
-  hipLaunchKernelGGL(GroupRouteKernel, dim3(1), dim3(kRouteThreads), GroupedRouteLds(gp.G), stream, gp);
   mg::GemmArgs g{};
   g.A = p.g.A;
   g.B = p.X;
@@ -273,13 +273,23 @@ void LaunchDqGroupedMatMul(const DqGroupedParams &p, hipStream_t stream) {
   g.scale_f16 = p.scale_f16;
   g.scale_per_col = p.scale_per_col;
   g.scale_grp_stride = p.scale_grp_stride;
-  g.grp_tile_off = p.g.tile_off;
-  g.grp_row_off = p.g.row_off;
-  g.grp_rows = p.g.rows;
   g.grp_count = (int)p.g.G;
   g.grp_sel = (int)p.g.S;
   g.grp_b_stride = p.g.K * p.g.N;
   g.grp_bias = p.g.bias;
+  if (sk::PrefersSkinnyGrouped(g)) {  // one launch, no routing pass
+    LaunchF8SkinnyGrouped(g, p.g.idx, p.g.idx64, stream);
+    return;
+  }
+  // 256 x 256 tiles (as configuration 4's fp8 GEMM) when K takes whole K
+  // steps; the routing then counts 256-column tiles
+  GroupedParams gp = p.g;
+  const bool wide = p.g.K % 64 == 0;
+  if (wide) gp.nbn = (p.g.N + 255) / 256;
+  hipLaunchKernelGGL(GroupRouteKernel, dim3(1), dim3(kRouteThreads), GroupedRouteLds(gp.G), stream, gp);
+  g.grp_tile_off = p.g.tile_off;
+  g.grp_row_off = p.g.row_off;
+  g.grp_rows = p.g.rows;
   if (wide) mg::LaunchGrouped<mg::kOutBf16, 1, mg::kBf16F8, 4>(g, GroupedMaxTiles(gp), stream);
   else mg::LaunchGrouped<mg::kOutBf16, 1, mg::kBf16F8, 2>(g, GroupedMaxTiles(gp), stream);
 }

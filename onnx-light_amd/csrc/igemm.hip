@@ -5,14 +5,17 @@
 //    outputs to fill the chip: the pipelined core (mfma_gemm.hpp).
 //  - every other shape or alignment, and fewer outputs: the small-tile GEMM
 //    (tile_gemm.hpp, where the line is drawn and measured).
+//  - a few rows (decode): skinny_gemm.hpp, likewise.
 #include "common.hpp"
 #include "kernels.hpp"
 #include "igemm_fast.hpp"
+#include "skinny_gemm.hpp"
 #include "tile_gemm.hpp"
 
 namespace onnxl_amd {
 
 void LaunchIGemmTile(const IGemmParams &p, bool big, hipStream_t s);
+void LaunchIGemmSkinny(const IGemmParams &p, hipStream_t s);
 
 void LaunchIGemm(const IGemmParams &p, hipStream_t stream) {
   if (p.M == 0 || p.N == 0 || p.batch == 0) return;
@@ -23,6 +26,10 @@ void LaunchIGemm(const IGemmParams &p, hipStream_t stream) {
     return;
   }
   const mg::GemmArgs g = ToGemmArgs(p);
+  if (p.epilogue != kEpiQuant8Row && sk::PrefersSkinny(g, true, p.need_ra || p.need_cb)) {
+    LaunchIGemmSkinny(p, stream);
+    return;
+  }
   const bool small = tg::PrefersSmallTile(g);
   if (small || !mg::Eligible<mg::kI8>(g)) {
     LaunchIGemmTile(p, !small, stream);
