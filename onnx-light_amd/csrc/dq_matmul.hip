@@ -124,7 +124,8 @@ void LaunchFp8Gemm(const mg::GemmArgs &g, hipStream_t stream) {
   const int64_t cus = DeviceCUs();
   const int64_t nbm = (g.M + 255) / 256, nbn = (g.N + 255) / 256;
   if (nbm * nbn < 512 || g.K % 64 != 0) {  // 256 x 256 tiles take whole K steps only
-    mg::Launch<mg::kBf16F8, mg::kOutBf16, false, false, false, 2>(g, stream);
+    if (mg::PrefersHalfTile<mg::kBf16F8>(g)) mg::Launch<mg::kBf16F8, mg::kOutBf16, false, false, false, 2, false, 2>(g, stream);
+    else mg::Launch<mg::kBf16F8, mg::kOutBf16, false, false, false, 2>(g, stream);
     return;
   }
   int64_t nb = nbn;  // tile-columns in 256 x 256 tiles
@@ -172,8 +173,11 @@ mg::GemmArgs Fp8Args(const DqMatMulParams &p) {
 void LaunchHMatMul(const HMatMulParams &p, hipStream_t stream) {
   if (p.M == 0 || p.N == 0 || p.batch == 0) return;
   const mg::GemmArgs g = HArgs(p);
-  const bool small = tg::PrefersSmallTile(g);
-  if (small || !mg::Eligible<mg::kH16>(g)) LaunchHTile(g, p.bf16, !small, stream);
+  const bool core = mg::Eligible<mg::kH16>(g), small = tg::PrefersSmallTile(g, core);
+  const bool half = mg::PrefersHalfTile<mg::kH16>(g);
+  if (small || !core) LaunchHTile(g, p.bf16, !small, stream);
+  else if (half && p.bf16) mg::Launch<mg::kH16, mg::kOutBf16, false, false, false, 2, false, 2>(g, stream);
+  else if (half) mg::Launch<mg::kH16, mg::kOutF16, false, false, false, 2, false, 2>(g, stream);
   else if (p.bf16) mg::Launch<mg::kH16, mg::kOutBf16, false, false, false>(g, stream);
   else mg::Launch<mg::kH16, mg::kOutF16, false, false, false>(g, stream);
 }
@@ -184,8 +188,11 @@ void LaunchHMatMulBT(const HMatMulParams &p, hipStream_t stream) {
   const mg::GemmArgs g = HArgs(p);
   if (p.N % 16 != 0 && p.M > 65535)
     throw Unsupported("MatMul with B given as [N, K]: N % 16 != 0 takes at most 65535 rows");
-  const bool small = tg::PrefersSmallTile(g);
-  if (small || !mg::EligibleBT(g)) LaunchHTileBT(g, p.bf16, !small, stream);
+  const bool core = mg::EligibleBT(g), small = tg::PrefersSmallTile(g, core);
+  const bool half = mg::PrefersHalfTile<mg::kH16>(g);
+  if (small || !core) LaunchHTileBT(g, p.bf16, !small, stream);
+  else if (half && p.bf16) mg::LaunchBT<mg::kOutBf16, 2>(g, stream);
+  else if (half) mg::LaunchBT<mg::kOutF16, 2>(g, stream);
   else if (p.bf16) mg::LaunchBT<mg::kOutBf16>(g, stream);
   else mg::LaunchBT<mg::kOutF16>(g, stream);
 }
@@ -215,7 +222,7 @@ bool LaunchDqMatMul(const DqMatMulParams &p, void *scratch, size_t scratch_bytes
   }
   if (Fp8Eligible(p)) {
     const mg::GemmArgs g = Fp8Args(p);
-    const bool core = mg::Eligible<mg::kBf16F8>(g), small = tg::PrefersSmallTile(g);
+    const bool core = mg::Eligible<mg::kBf16F8>(g), small = tg::PrefersSmallTile(g, core);
     if (core && sk::PrefersSkinny(g, false, false)) LaunchF8Skinny(g, stream);
     else if (core && !small) LaunchFp8Gemm(g, stream);
     else LaunchF8Tile(g, /*chain=*/!core, !small, stream);

@@ -59,13 +59,13 @@ __global__ __launch_bounds__(kRouteThreads) void GroupRouteKernel(const GroupedP
   }
   __syncthreads();
   // exclusive scans of the row counts and of the tile counts
-  // (ceil(rows / 256) tile-rows of nbn tiles)
+  // (ceil(rows / tile_rows) tile-rows of nbn tiles)
   const int per = (G + kRouteThreads - 1) / kRouteThreads;
   const int g0 = tid * per, g1 = min(G, g0 + per);
   int32_t rs = 0, ts = 0;
   for (int g = g0; g < g1; ++g) {
     rs += cnt[g];
-    ts += (cnt[g] + mg::kBM - 1) / mg::kBM * p.nbn;
+    ts += (cnt[g] + p.tile_rows - 1) / p.tile_rows * p.nbn;
   }
   rsum[tid] = rs;
   tsum[tid] = ts;
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(kRouteThreads) void GroupRouteKernel(const GroupedP
     p.tile_off[g] = trun;
     cursor[g] = rrun;
     rrun += cnt[g];
-    trun += (cnt[g] + mg::kBM - 1) / mg::kBM * p.nbn;
+    trun += (cnt[g] + p.tile_rows - 1) / p.tile_rows * p.nbn;
   }
   if (tid == kRouteThreads - 1) {
     p.row_off[G] = rsum[tid];
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(256) void DequantExpertsKernel(const DqGroupedParam
 }  // namespace
 
 int64_t GroupedMaxTiles(const GroupedParams &p) {
-  return ((p.M * p.S + mg::kBM - 1) / mg::kBM + p.G) * p.nbn;
+  return ((p.M * p.S + p.tile_rows - 1) / p.tile_rows + p.G) * p.nbn;
 }
 
 size_t GroupedRouteLds(int64_t G) { return (size_t)(2 * G) * sizeof(int32_t); }
@@ -192,9 +192,32 @@ bool GroupedCoreEligible(const GroupedParams &p) {
          (p.bias == nullptr || reinterpret_cast<uintptr_t>(p.bias) % 8 == 0);
 }
 
-void LaunchGroupedMatMul(const GroupedParams &p, hipStream_t stream) {
+namespace {
+
+// Rounds of the chip that a grouped launch of r x c tiles takes.  The host does
+// not know the groups' sizes: every group is taken a tenth larger than the
+// average, since a few rows past a multiple of r cost a whole tile row.
+int64_t GroupedRounds(const GroupedParams &p, int64_t r, int64_t c) {
+  const int64_t avg = (p.M * p.S + p.G - 1) / p.G, rows = avg + avg / 10;
+  return mg::Rounds(p.G * ((rows + r - 1) / r) * ((p.N + c - 1) / c));
+}
+
+template <int OUT, int GM> void LaunchGroupedCore(const mg::GemmArgs &g, int64_t tiles, bool half, hipStream_t s) {
+  if (half) mg::LaunchGrouped<OUT, GM, mg::kH16, 2, 2>(g, tiles, s);
+  else mg::LaunchGrouped<OUT, GM>(g, tiles, s);
+}
+
+}  // namespace
+
+void LaunchGroupedMatMul(const GroupedParams &gp, hipStream_t stream) {
+  GroupedParams p = gp;
   const int64_t P = p.M * p.S;
   if (P == 0 || p.N == 0) return;
+  // 128-row tiles where they take less than 20 / 12 of the 256-row ones' rounds
+  // (as PrefersHalfTile; bf16, 4 experts [4096, 4096] given [N, K], top-2: 256
+  // tokens 46.5 -> 36.6 us, 500 tokens 51.2 against 62.5 us)
+  const bool half = 12 * GroupedRounds(p, 128, 128) < 20 * GroupedRounds(p, 256, 128);
+  p.tile_rows = half ? 128 : 256;
   hipLaunchKernelGGL(GroupRouteKernel, dim3(1), dim3(kRouteThreads), GroupedRouteLds(p.G), stream, p);
   if (p.K == 0 || !GroupedCoreEligible(p)) {
     const int64_t items = (p.N + 255) / 256 * P;
@@ -219,11 +242,11 @@ void LaunchGroupedMatMul(const GroupedParams &p, hipStream_t stream) {
   g.grp_bias = p.bias;
   const int64_t tiles = GroupedMaxTiles(p);
   if (p.bf16) {
-    if (p.transB) mg::LaunchGrouped<mg::kOutBf16, 2>(g, tiles, stream);
-    else mg::LaunchGrouped<mg::kOutBf16, 1>(g, tiles, stream);
+    if (p.transB) LaunchGroupedCore<mg::kOutBf16, 2>(g, tiles, half, stream);
+    else LaunchGroupedCore<mg::kOutBf16, 1>(g, tiles, half, stream);
   } else {
-    if (p.transB) mg::LaunchGrouped<mg::kOutF16, 2>(g, tiles, stream);
-    else mg::LaunchGrouped<mg::kOutF16, 1>(g, tiles, stream);
+    if (p.transB) LaunchGroupedCore<mg::kOutF16, 2>(g, tiles, half, stream);
+    else LaunchGroupedCore<mg::kOutF16, 1>(g, tiles, half, stream);
   }
 }
 
@@ -281,17 +304,27 @@ void LaunchDqGroupedMatMul(const DqGroupedParams &p, hipStream_t stream) {
     LaunchF8SkinnyGrouped(g, p.g.idx, p.g.idx64, stream);
     return;
   }
-  // 256 x 256 tiles (as configuration 4's fp8 GEMM) when K takes whole K
-  // steps; the routing then counts 256-column tiles
+  // 128 x 128 tiles, or 256 x 256 ones (as configuration 4's fp8 GEMM) when K
+  // takes whole K steps; the routing then counts 256-column tiles.  A round of
+  // the former takes about 0.31 of the latter's time: fp8 experts, K = 4096,
+  // top-2, 256 x 256 -> 128 x 128: 8 x N = 4096, 256 tokens 81.0 -> 35.6 us, 2000
+  // tokens 182 -> 133 us; 8 x N = 14336, 256 tokens 169 -> 131 us, 1000 tokens 220
+  // against 247 us.
   GroupedParams gp = p.g;
-  const bool wide = p.g.K % 64 == 0;
+  const bool whole = p.g.K % 64 == 0;
+  const bool half = whole ? 10 * GroupedRounds(gp, 128, 128) < 32 * GroupedRounds(gp, 256, 256)
+                          : 11 * GroupedRounds(gp, 128, 128) < 20 * GroupedRounds(gp, 256, 128);
+  const bool wide = whole && !half;
   if (wide) gp.nbn = (p.g.N + 255) / 256;
+  gp.tile_rows = half ? 128 : 256;
   hipLaunchKernelGGL(GroupRouteKernel, dim3(1), dim3(kRouteThreads), GroupedRouteLds(gp.G), stream, gp);
   g.grp_tile_off = p.g.tile_off;
   g.grp_row_off = p.g.row_off;
   g.grp_rows = p.g.rows;
-  if (wide) mg::LaunchGrouped<mg::kOutBf16, 1, mg::kBf16F8, 4>(g, GroupedMaxTiles(gp), stream);
-  else mg::LaunchGrouped<mg::kOutBf16, 1, mg::kBf16F8, 2>(g, GroupedMaxTiles(gp), stream);
+  const int64_t tiles = GroupedMaxTiles(gp);
+  if (half) mg::LaunchGrouped<mg::kOutBf16, 1, mg::kBf16F8, 2, 2>(g, tiles, stream);
+  else if (wide) mg::LaunchGrouped<mg::kOutBf16, 1, mg::kBf16F8, 4>(g, tiles, stream);
+  else mg::LaunchGrouped<mg::kOutBf16, 1, mg::kBf16F8, 2>(g, tiles, stream);
 }
 
 }  // namespace onnxl_amd

@@ -19,27 +19,23 @@ void LaunchIGemmSkinny(const IGemmParams &p, hipStream_t s);
 
 void LaunchIGemm(const IGemmParams &p, hipStream_t stream) {
   if (p.M == 0 || p.N == 0 || p.batch == 0) return;
+  const mg::GemmArgs g = ToGemmArgs(p);
+  const bool half = mg::PrefersHalfTile<mg::kI8>(g);
   if (p.implicit_conv) {  // the caller checked the implicit operand's shape
-    if (p.epilogue == kEpiInt32) LaunchIGemmConvI32(p, stream);
-    else if (p.epilogue == kEpiQuant8Row) LaunchIGemmConvQ8Row(p, stream);
+    if (p.epilogue == kEpiInt32) LaunchIGemmConvI32(p, half, stream);
+    else if (p.epilogue == kEpiQuant8Row) LaunchIGemmConvQ8Row(p, half, stream);
     else throw DeviceError("internal: implicit convolution with a per-tensor requantization");
     return;
   }
-  const mg::GemmArgs g = ToGemmArgs(p);
   if (p.epilogue != kEpiQuant8Row && sk::PrefersSkinny(g, true, p.need_ra || p.need_cb)) {
     LaunchIGemmSkinny(p, stream);
     return;
   }
-  const bool small = tg::PrefersSmallTile(g);
-  if (small || !mg::Eligible<mg::kI8>(g)) {
-    LaunchIGemmTile(p, !small, stream);
-  } else if (p.epilogue == kEpiInt32) {
-    LaunchIGemmFastI32(p, stream);
-  } else if (p.epilogue == kEpiQuant8Row) {
-    LaunchIGemmFastQ8Row(p, stream);
-  } else {
-    LaunchIGemmFastQ8(p, stream);
-  }
+  const bool core = mg::Eligible<mg::kI8>(g), small = tg::PrefersSmallTile(g, core);
+  if (small || !core) LaunchIGemmTile(p, !small, stream);
+  else if (p.epilogue == kEpiInt32) LaunchIGemmFastI32(p, half, stream);
+  else if (p.epilogue == kEpiQuant8Row) LaunchIGemmFastQ8Row(p, half, stream);
+  else LaunchIGemmFastQ8(p, half, stream);
 }
 
 

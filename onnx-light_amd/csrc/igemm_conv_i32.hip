@@ -3,5 +3,5 @@
 #include "igemm_fast.hpp"
 
 namespace onnxl_amd {
-void LaunchIGemmConvI32(const IGemmParams &p, hipStream_t s) { LaunchIGemmFastOut<mg::kOutI32, true>(p, s); }
+void LaunchIGemmConvI32(const IGemmParams &p, bool half, hipStream_t s) { LaunchIGemmFastOut<mg::kOutI32, true>(p, half, s); }
 }  // namespace onnxl_amd

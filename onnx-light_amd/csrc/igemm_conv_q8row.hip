@@ -3,5 +3,5 @@
 #include "igemm_fast.hpp"
 
 namespace onnxl_amd {
-void LaunchIGemmConvQ8Row(const IGemmParams &p, hipStream_t s) { LaunchIGemmFastOut<mg::kOutQ8Row, true>(p, s); }
+void LaunchIGemmConvQ8Row(const IGemmParams &p, bool half, hipStream_t s) { LaunchIGemmFastOut<mg::kOutQ8Row, true>(p, half, s); }
 }  // namespace onnxl_amd

@@ -41,26 +41,32 @@ inline mg::GemmArgs ToGemmArgs(const IGemmParams &p) {
 
 // Row / column sums are accumulated only when a zero point makes them count.
 // CV: B is an implicit convolution operand (p.implicit_conv).
-template <int OUT, bool CV = false> void LaunchIGemmFastOut(const IGemmParams &p, hipStream_t s) {
+template <int OUT, bool CV, int MB> void LaunchIGemmFastTile(const IGemmParams &p, hipStream_t s) {
   const mg::GemmArgs g = ToGemmArgs(p);
   const bool zp = p.need_ra || p.need_cb;
   const int sel = (zp ? 4 : 0) | (p.a_u8 ? 2 : 0) | (p.b_u8 ? 1 : 0);
   switch (sel) {
-  case 0: mg::Launch<mg::kI8, OUT, false, false, false, 2, CV>(g, s); break;
-  case 1: mg::Launch<mg::kI8, OUT, false, false, true, 2, CV>(g, s); break;
-  case 2: mg::Launch<mg::kI8, OUT, false, true, false, 2, CV>(g, s); break;
-  case 3: mg::Launch<mg::kI8, OUT, false, true, true, 2, CV>(g, s); break;
-  case 4: mg::Launch<mg::kI8, OUT, true, false, false, 2, CV>(g, s); break;
-  case 5: mg::Launch<mg::kI8, OUT, true, false, true, 2, CV>(g, s); break;
-  case 6: mg::Launch<mg::kI8, OUT, true, true, false, 2, CV>(g, s); break;
-  default: mg::Launch<mg::kI8, OUT, true, true, true, 2, CV>(g, s); break;
+  case 0: mg::Launch<mg::kI8, OUT, false, false, false, 2, CV, MB>(g, s); break;
+  case 1: mg::Launch<mg::kI8, OUT, false, false, true, 2, CV, MB>(g, s); break;
+  case 2: mg::Launch<mg::kI8, OUT, false, true, false, 2, CV, MB>(g, s); break;
+  case 3: mg::Launch<mg::kI8, OUT, false, true, true, 2, CV, MB>(g, s); break;
+  case 4: mg::Launch<mg::kI8, OUT, true, false, false, 2, CV, MB>(g, s); break;
+  case 5: mg::Launch<mg::kI8, OUT, true, false, true, 2, CV, MB>(g, s); break;
+  case 6: mg::Launch<mg::kI8, OUT, true, true, false, 2, CV, MB>(g, s); break;
+  default: mg::Launch<mg::kI8, OUT, true, true, true, 2, CV, MB>(g, s); break;
   }
 }
 
-void LaunchIGemmFastI32(const IGemmParams &p, hipStream_t s);
-void LaunchIGemmFastQ8(const IGemmParams &p, hipStream_t s);
-void LaunchIGemmFastQ8Row(const IGemmParams &p, hipStream_t s);
-void LaunchIGemmConvI32(const IGemmParams &p, hipStream_t s);
-void LaunchIGemmConvQ8Row(const IGemmParams &p, hipStream_t s);
+// half: 128-row tiles instead of 256-row ones.
+template <int OUT, bool CV = false> void LaunchIGemmFastOut(const IGemmParams &p, bool half, hipStream_t s) {
+  if (half) LaunchIGemmFastTile<OUT, CV, 2>(p, s);
+  else LaunchIGemmFastTile<OUT, CV, 4>(p, s);
+}
+
+void LaunchIGemmFastI32(const IGemmParams &p, bool half, hipStream_t s);
+void LaunchIGemmFastQ8(const IGemmParams &p, bool half, hipStream_t s);
+void LaunchIGemmFastQ8Row(const IGemmParams &p, bool half, hipStream_t s);
+void LaunchIGemmConvI32(const IGemmParams &p, bool half, hipStream_t s);
+void LaunchIGemmConvQ8Row(const IGemmParams &p, bool half, hipStream_t s);
 
 }  // namespace onnxl_amd

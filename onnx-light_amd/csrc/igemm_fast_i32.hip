@@ -2,5 +2,5 @@
 #include "igemm_fast.hpp"
 
 namespace onnxl_amd {
-void LaunchIGemmFastI32(const IGemmParams &p, hipStream_t s) { LaunchIGemmFastOut<mg::kOutI32>(p, s); }
+void LaunchIGemmFastI32(const IGemmParams &p, bool half, hipStream_t s) { LaunchIGemmFastOut<mg::kOutI32>(p, half, s); }
 }  // namespace onnxl_amd

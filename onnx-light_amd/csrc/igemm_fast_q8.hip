@@ -2,5 +2,5 @@
 #include "igemm_fast.hpp"
 
 namespace onnxl_amd {
-void LaunchIGemmFastQ8(const IGemmParams &p, hipStream_t s) { LaunchIGemmFastOut<mg::kOutQ8>(p, s); }
+void LaunchIGemmFastQ8(const IGemmParams &p, bool half, hipStream_t s) { LaunchIGemmFastOut<mg::kOutQ8>(p, half, s); }
 }  // namespace onnxl_amd

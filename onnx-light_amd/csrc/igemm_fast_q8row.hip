@@ -3,5 +3,5 @@
 #include "igemm_fast.hpp"
 
 namespace onnxl_amd {
-void LaunchIGemmFastQ8Row(const IGemmParams &p, hipStream_t s) { LaunchIGemmFastOut<mg::kOutQ8Row>(p, s); }
+void LaunchIGemmFastQ8Row(const IGemmParams &p, bool half, hipStream_t s) { LaunchIGemmFastOut<mg::kOutQ8Row>(p, half, s); }
 }  // namespace onnxl_amd

@@ -451,6 +451,7 @@ struct GroupedParams {
   int64_t M, K, N, G, S;
   int idx64, transB, bf16;
   int64_t nbn;       // column tiles of the GEMM core: ceil(N / 128)
+  int tile_rows;     // rows of its tiles, set by the launchers
   // device workspace: G + 1, G + 1 and M * S int32
   int32_t *row_off, *tile_off, *rows;
 };

@@ -69,7 +69,6 @@ typedef __attribute__((address_space(3))) v4s *lds_v4s_t;
 
 constexpr int kBM = 256, kStepBytes = 128, kStages = 3, kThreads = 256;
 constexpr int kGroupM = 4, kXcds = 8;
-constexpr int kAStage = kBM * kStepBytes;  // 32 KB
 constexpr int kRsrcWord3 = 0x00020000;
 constexpr unsigned kOob = 0x80000000u;
 constexpr unsigned kFlip = 0x80808080u;
@@ -120,8 +119,7 @@ template <> struct Traits<kH16> {
 // halves the operand bytes per MFMA and fills the 256 accumulator registers).
 template <int KIND, int WB> constexpr int BPitch() { return 64 * WB * Traits<KIND>::kBsz; }
 template <int KIND, int WB> constexpr int BStageBytes() { return Traits<KIND>::kBRows * BPitch<KIND, WB>(); }
-// direct loads per wave per K step: A 32 KB + B stage, 1 KB per instruction
-template <int KIND, int WB> constexpr int LoadsPerWave() { return (kAStage + BStageBytes<KIND, WB>()) / 1024 / 4; }
+// direct loads of B per wave per K step, 1 KB per instruction
 template <int KIND, int WB> constexpr int BLoadsPerWave() { return BStageBytes<KIND, WB>() / 1024 / 4; }
 
 __device__ __forceinline__ int64_t MinI64(int64_t a, int64_t b) { return a < b ? a : b; }
@@ -229,8 +227,14 @@ __device__ __forceinline__ uint32_t DivMagic(uint32_t x, uint32_t magic) {
 // CV: implicit convolution (int8): B is read like A, its row for output
 // position n and K step t at the byte offset of GemmArgs::cv, so the im2col
 // matrix is never written.
-template <int KIND, int OUT, bool ZP, bool AU8, bool BU8, int WB, int GM = 0, bool CV = false>
-__global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) {
+//
+// MB: 32-row blocks per wave.  4 is the 256-row tile; 2 halves it (128 rows),
+// for problems whose 256-row tiles leave CUs idle.
+template <int KIND, int OUT, bool ZP, bool AU8, bool BU8, int WB, int GM = 0, bool CV = false, int MB = 4>
+__global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void MfmaGemmKernel(const GemmArgs p) {
+  constexpr int BM = 64 * MB, AST = BM * kStepBytes;  // tile rows, bytes of an A stage
+  constexpr int LA = AST / 1024 / 4;                  // direct loads of A per wave per K step
+  static_assert(MB == 4 || (MB == 2 && WB == 2), "tile height");
   constexpr bool RA = ZP, CB = ZP;
   constexpr bool GRP = GM == 1 || GM == 2;  // grouped (routing tables)
   constexpr bool BT = GM == 2 || GM == 3 || CV;
@@ -250,14 +254,13 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
   // different positions, where the plain one put them on 8 twice.
   constexpr int kBSwz = kBP >= 256 ? 2 : 1;
   constexpr int kBStage = BStageBytes<KIND, WB>();
-  constexpr int L = LoadsPerWave<KIND, WB>();
-  constexpr int LB = BLoadsPerWave<KIND, WB>();
+  constexpr int LB = BLoadsPerWave<KIND, WB>(), L = LA + LB;
   static_assert(WB == 2 || (WB == 4 && KIND != kH16), "tile width");
   constexpr int kOsz = OUT == kOutI32 ? 4 : (OUT == kOutQ8 || OUT == kOutQ8Row ? 1 : 2);
   static_assert(LB >= 1 && LB <= 4, "B direct loads per wave");
   // One object per ring stage: the compiler's LDS-DMA wait tracking can then
   // tell a read of one stage from a direct load into another.
-  __shared__ __align__(16) char sa0[kAStage], sa1[kAStage], sa2[kAStage];
+  __shared__ __align__(16) char sa0[AST], sa1[AST], sa2[AST];
   __shared__ __align__(16) char sb0[kBStage], sb1[kBStage], sb2[kBStage];
   __shared__ int32_t zsum[ZP ? (kThreads / 64) * 2 * kWN : 1];  // per wave: CB and beta of its columns
   __shared__ __align__(16) float cscale[KIND == kBf16F8 ? (kThreads / 64) * kWN : 4];  // per wave: column scales
@@ -304,13 +307,13 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
     const int64_t local = t - p.grp_tile_off[grp];
     rbase = p.grp_row_off[grp];
     rcount = p.grp_row_off[grp + 1] - rbase;
-    const int64_t nbm = (rcount + kBM - 1) / kBM;
+    const int64_t nbm = (rcount + BM - 1) / BM;
     const int64_t first_m = local / (kGroupM * nbn) * kGroupM;
     const int64_t gsize = MinI64(nbm - first_m, kGroupM);
-    row0 = (first_m + (local % (kGroupM * nbn)) % gsize) * kBM;
+    row0 = (first_m + (local % (kGroupM * nbn)) % gsize) * BM;
     col0 = (local % (kGroupM * nbn)) / gsize * kBN;
   } else {
-    const int64_t nbm = (M + kBM - 1) / kBM;
+    const int64_t nbm = (M + BM - 1) / BM;
     const int64_t tiles = nbm * nbn;
     const int64_t total = tiles * p.batch;
     const int64_t pid = blockIdx.x;
@@ -323,7 +326,7 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
     const int64_t gsize = MinI64(nbm - first_m, kGroupM);
     const int64_t tm = first_m + (tt % (kGroupM * nbn)) % gsize;
     const int64_t tn = (tt % (kGroupM * nbn)) / gsize;
-    row0 = tm * kBM;
+    row0 = tm * BM;
     col0 = tn * kBN;
   }
 
@@ -353,10 +356,10 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
   const int nk = nfull + (half ? 1 : 0);                    // K steps to load
 
   // ---- direct-load offsets (K step 0) ----
-  unsigned a_g[8];
+  unsigned a_g[8];  // LA <= 8
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int64_t row = row0 + 8 * (8 * wave + q) + (lane >> 3);  // 8-row block 8 * wave + q
+  for (int q = 0; q < LA; ++q) {
+    const int64_t row = row0 + 8 * (LA * wave + q) + (lane >> 3);  // 8-row block LA * wave + q
     int64_t src = row;  // row of A
     if constexpr (GRP) src = row < rcount ? p.grp_rows[rbase + row] / p.grp_sel : 0;
     a_g[q] = row < rcount ? (unsigned)(src * KA + 16 * ((lane & 7) ^ (lane >> 3) ^ (q & 1))) : kOob;
@@ -390,13 +393,13 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
     }
   }
   // ---- LDS fragment offsets (sub-step 0; sub-step kk adds kk * const) ----
-  // Sub-step kk reads chunk 2 kk + lg of row wm * 128 + 32 i + lr; block i
+  // Sub-step kk reads chunk 2 kk + lg of row wm * 32 MB + 32 i + lr; block i
   // sits exactly 4096 bytes after block i-1, so one base per sub-step serves
-  // all four blocks through the DS offset field.
+  // all blocks through the DS offset field.
   int a_rd[4];
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk)
-    a_rd[kk] = (wm * 128 + lr) * 128 + 16 * ((2 * kk + lg) ^ (lr & 7) ^ ((lr >> 3) & 1));
+    a_rd[kk] = (wm * 32 * MB + lr) * 128 + 16 * ((2 * kk + lg) ^ (lr & 7) ^ ((lr >> 3) & 1));
   const int s16 = lane & 15, g16 = lane >> 4;
   // One base per column block j; the second transposing read of a fragment
   // (h = 1) is 8 rows (int8) or 4 rows (16-bit) further, the same swizzle.
@@ -441,15 +444,15 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
                               : static_cast<const float *>(p.scale)[si];
     }
   }
-  // kOutQ8Row: the weight scale and bias of this lane's rows in the four
+  // kOutQ8Row: the weight scale and bias of this lane's rows in the
   // 32-row blocks, loaded here so that their latency hides under the K loop
   // instead of opening each block's epilogue
-  float row_ws[OUT == kOutQ8Row ? 4 : 1] = {};
-  int32_t row_b[OUT == kOutQ8Row ? 4 : 1] = {};
+  float row_ws[OUT == kOutQ8Row ? MB : 1] = {};
+  int32_t row_b[OUT == kOutQ8Row ? MB : 1] = {};
   if constexpr (OUT == kOutQ8Row) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int64_t row = row0 + wm * 128 + i * 32 + lr;
+    for (int i = 0; i < MB; ++i) {
+      const int64_t row = row0 + wm * 32 * MB + i * 32 + lr;
       const int64_t rc = row < M ? row : 0;
       row_ws[i] = p.row_wscale[p.row_wscale_per ? rc : 0];
       row_b[i] = p.row_bias ? p.row_bias[rc] : 0;
@@ -459,7 +462,7 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
   constexpr int bflip = (KIND == kI8 && BU8) ? (int)kFlip : 0;
 
   // Direct loads of K step `step` into ring stage `stage`: the L loads of a
-  // step, numbered A pieces 0..7 then B pieces, in quarters (parts 0..3) or
+  // step, numbered A pieces then B pieces, in quarters (parts 0..3) or
   // all at once (part 4).
   auto issue = [&](int step, int stage, int part) __attribute__((always_inline)) {
     const bool live = step < nk;
@@ -477,12 +480,12 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
     const __amdgpu_buffer_rsrc_t rsa = live ? rsA : rsA0, rsb = live ? rsB : rsB0;
     const int lo = part == 4 ? 0 : part * L / 4, hi = part == 4 ? L : (part + 1) * L / 4;
 #pragma unroll
-    for (int q = 0; q < 8; ++q)
+    for (int q = 0; q < LA; ++q)
       if (q >= lo && q < hi)
-        DirectLoad16(rsa, sa + (8 * wave + q) * 1024, a_g[q] + ka);
+        DirectLoad16(rsa, sa + (LA * wave + q) * 1024, a_g[q] + ka);
 #pragma unroll
     for (int q = 0; q < LB; ++q)
-      if (8 + q >= lo && 8 + q < hi)
+      if (LA + q >= lo && LA + q < hi)
         DirectLoad16(rsb, sb + (wave * LB + q) * 1024, b_g[q] + kb);
   };
 
@@ -492,7 +495,7 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
   // LDS reads were issued two sub-steps earlier and the fp8 decode ran under
   // the MFMAs of sub-step s - 1, so neither the LDS latency nor the decode
   // VALU work stalls the matrix pipe.
-  v4i ra[3][4];
+  v4i ra[3][MB];
   v4i rb[3][WB];  // raw B: kI8 2 x tr8; kBf16F8 1 x tr8 (.xy); kH16 2 x tr16
   auto read = [&](int buf, const char *sa, const char *sb, int kk) __attribute__((always_inline)) {
 #pragma unroll
@@ -515,16 +518,16 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
       }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MB; ++i)
       ra[buf][i] = *reinterpret_cast<const v4i *>(sa + a_rd[kk] + i * 4096);
   };
 
-  Acc acc[4][WB];
+  Acc acc[MB][WB];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < WB; ++j) acc[i][j] = Acc{0};
-  int rsum[4] = {0, 0, 0, 0};  // kI8: partial row sums of a' (this lane's k group)
+  int rsum[MB] = {};  // kI8: partial row sums of a' (this lane's k group)
   int csum[WB];                // kI8: partial column sums of b'
 #pragma unroll
   for (int j = 0; j < WB; ++j) csum[j] = 0;
@@ -539,7 +542,7 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
   auto decode = [&](int rbuf, int bbuf) __attribute__((always_inline)) {
     if constexpr (KIND == kI8 && AU8) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) ra[rbuf][i] ^= aflip;
+      for (int i = 0; i < MB; ++i) ra[rbuf][i] ^= aflip;
     }
 #pragma unroll
     for (int j = 0; j < WB; ++j) {
@@ -596,15 +599,15 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
 
   // Instruction order inside a sub-step, pinned because the scheduler would
   // otherwise sink each LDS read next to its first use.
-  constexpr int kReads = 4 + WB * (KIND == kBf16F8 ? 1 : 2);
-  constexpr int kDecodeValu = KIND == kBf16F8 ? 4 * WB : (KIND == kI8 ? (AU8 ? 16 : 0) + (BU8 ? 4 * WB : 0) + (CB ? 4 * WB : 0) : 0);
+  constexpr int kReads = MB + WB * (KIND == kBf16F8 ? 1 : 2);
+  constexpr int kDecodeValu = KIND == kBf16F8 ? 4 * WB : (KIND == kI8 ? (AU8 ? 4 * MB : 0) + (BU8 ? 4 * WB : 0) + (CB ? 4 * WB : 0) : 0);
   // A plain sub-step with `nvm` direct loads: each MFMA is preceded by its
   // share of the LDS reads two sub-steps ahead and followed by a direct load
   // and its share of the decode.  Reads issued all at once at the top of a
   // sub-step (4 waves x 8 reads) queue up in the LDS; one read per MFMA cost
   // 9% fewer cycles on C2.
   auto order_vm = [&](int nvm) __attribute__((always_inline)) {
-    constexpr int kNM = 4 * WB;
+    constexpr int kNM = MB * WB;
 #pragma unroll
     for (int x = 0; x < kNM; ++x) {
       __builtin_amdgcn_sched_group_barrier(0x100, (kReads + kNM - 1) / kNM, 0);  // DS read
@@ -616,14 +619,15 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
   };
   // second half of the barrier sub-step with `nvm` direct loads
   auto order_refill = [&](int nvm) __attribute__((always_inline)) {
+    constexpr int kHM = MB / 2 * WB;
 #pragma unroll
-    for (int x = 0; x < 2 * WB; ++x) {
-      __builtin_amdgcn_sched_group_barrier(0x100, (kReads + 2 * WB - 1) / (2 * WB), 0);  // DS read
+    for (int x = 0; x < kHM; ++x) {
+      __builtin_amdgcn_sched_group_barrier(0x100, (kReads + kHM - 1) / (kHM), 0);  // DS read
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);               // MFMA
       if (x < nvm) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // VMEM
-      if (x + 2 * WB < nvm) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      if (x + kHM < nvm) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
       if constexpr (kDecodeValu > 0)
-        __builtin_amdgcn_sched_group_barrier(0x002, (kDecodeValu + 2 * WB - 1) / (2 * WB), 0);  // VALU
+        __builtin_amdgcn_sched_group_barrier(0x002, (kDecodeValu + kHM - 1) / (kHM), 0);  // VALU
     }
   };
   // direct loads in refill quarter `part`
@@ -648,18 +652,18 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
       else issue(t + 2, prv, 2 + kk);
       decode(nb3, nb2);
       colsum(sb3);
-      mma(sb3, sb2, 0, 4);
+      mma(sb3, sb2, 0, MB);
       order_vm(kk == 3 ? quarter(1) : quarter(2 + kk));
       __builtin_amdgcn_sched_barrier(0);
     } else {
-      mma(sb3, sb2, 0, 2);
+      mma(sb3, sb2, 0, MB / 2);
       __builtin_amdgcn_sched_barrier(0);
       RingBarrier<L>();
       read(rb3, SA(nxt), SB(nxt), 0);
       issue(t + 3, cur, 0);  // first quarter of the refill
       decode(nb3, nb2);
       colsum(sb3);
-      mma(sb3, sb2, 2, 4);
+      mma(sb3, sb2, MB / 2, MB);
       order_refill(quarter(0));
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -675,12 +679,12 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
     decode((r3 + 1) % 3, 1);
     colsum(r3);
     colsum((r3 + 1) % 3);
-    mma(r3, 0, 0, 4);
-    mma((r3 + 1) % 3, 1, 0, 4);
+    mma(r3, 0, 0, MB);
+    mma((r3 + 1) % 3, 1, 0, MB);
   };
 
   // Zero points of this lane's rows (32i + lr) and columns (32j + lr).
-  uint32_t za[4] = {0, 0, 0, 0}, zb[4] = {0, 0, 0, 0};  // raw zero-point bytes
+  uint32_t za[MB] = {}, zb[4] = {0, 0, 0, 0};  // raw zero-point bytes
   auto load_zp = [&]() __attribute__((always_inline)) {
     if constexpr (KIND == kI8 && ZP) {
       const __amdgpu_buffer_rsrc_t rsZa =
@@ -688,8 +692,8 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
       const __amdgpu_buffer_rsrc_t rsZb =
           __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(p.b_zp), (short)0, (int)(p.b_zp ? N : 0), kRsrcWord3);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int64_t row = row0 + wm * 128 + i * 32 + lr;
+      for (int i = 0; i < MB; ++i) {
+        const int64_t row = row0 + wm * 32 * MB + i * 32 + lr;
         za[i] = __builtin_amdgcn_raw_buffer_load_b8(rsZa, row < M ? (unsigned)row : kOob, 0, 0);
       }
 #pragma unroll
@@ -768,10 +772,10 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
   QResolved qv{p.alpha_scalar, p.beta_scalar, p.cs, p.zy};
   if constexpr (KIND == kI8) qv = ResolveQ(p.dev, p.a_u8, p.b_u8, p.y_signed, p.alpha_scalar, p.beta_scalar, p.cs, p.zy);
   int32_t *zc = zsum + (KIND == kI8 && ZP ? wave * 2 * kWN : 0);
-  int zrow[4] = {0, 0, 0, 0};
+  int zrow[MB] = {};
   if constexpr (KIND == kI8 && ZP) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MB; ++i)
       zrow[i] = p.a_zp ? (p.a_u8 ? 128 - (int)za[i] : -(int)(int8_t)za[i]) : qv.alpha;
 #pragma unroll
     for (int j = 0; j < WB; ++j) {
@@ -805,12 +809,16 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
   // Per 32-row block the wave packs those four values, stages the block in LDS
   // (row pitch padded by 16 bytes) and writes whole 16-byte row pieces.
   constexpr int kPitch = kWN * kOsz + 16;
-  static_assert(32 * kPitch <= 16384 && 2 * 16384 <= kAStage, "epilogue staging: 32 rows per wave, two waves per stage");
+  // Two waves share an A stage where that holds 32 staged rows of each, else
+  // each has an array of its own.
+  constexpr bool kShared = 2 * 32 * kPitch <= AST;
+  static_assert(32 * kPitch <= (kShared ? AST / 2 : (AST < kBStage ? AST : kBStage)), "epilogue staging");
   // Staging areas in ring stages 1 and 2: the block-major path (one half
   // step) loads only stage 0 and writes a block's outputs while the partner
   // wave (same wm) may still read its fragments from stage 0; the full path
   // has drained every stage behind a barrier.
-  char *stg = (wave >> 1 ? sa2 : sa1) + (wave & 1) * 16384;
+  char *stg = kShared ? (wave >> 1 ? sa2 : sa1) + (wave & 1) * (AST / 2)
+                      : (wave == 0 ? sa1 : wave == 1 ? sa2 : wave == 2 ? sb1 : sb2);
   // QLinearMatMul requantization constants (signed outputs biased by 128)
   const float q_bias = p.y_signed ? 128.f : 0.f;
   const float q_zy = qv.zy + q_bias, q_lo = p.qmin + q_bias, q_hi = p.qmax + q_bias;
@@ -935,7 +943,7 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
     constexpr int kChunksPerRow = kWN * kOsz / 16;
     // Branch-free stores: pieces outside the matrix get an offset past the
     // buffer, which the buffer store drops; all LDS reads issue first.
-    const int64_t brow = row0 + wm * 128 + i * 32;
+    const int64_t brow = row0 + wm * 32 * MB + i * 32;
     const int64_t ncol = N - (col0 + wn * kWN);
     const unsigned ybase = (unsigned)((brow * LDY + col0 + wn * kWN) * kOsz);
     // grouped mode: each staged row goes to its own row of Y
@@ -969,7 +977,7 @@ __global__ __launch_bounds__(kThreads, 1) void MfmaGemmKernel(const GemmArgs p) 
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < MB; ++i) {
     if (block_major) {
       mma(0, 0, i, i + 1);
       mma(1, 1, i, i + 1);
@@ -992,12 +1000,28 @@ template <int KIND> inline bool Eligible(const GemmArgs &p) {
          p.M * ldy * 4 < lim && (p.K + 3 * Traits<KIND>::kKStep) * ldb * kBsz < lim;
 }
 
-template <int KIND, int OUT, bool ZP, bool AU8, bool BU8, int WB = 2, bool CV = false>
+template <int KIND, int OUT, bool ZP, bool AU8, bool BU8, int WB = 2, bool CV = false, int MB = 4>
 inline void Launch(const GemmArgs &p, hipStream_t s) {
   constexpr int kBN = 64 * WB;
-  const int64_t tiles = ((p.M + kBM - 1) / kBM) * ((p.N + kBN - 1) / kBN) * p.batch;
-  hipLaunchKernelGGL((MfmaGemmKernel<KIND, OUT, ZP, AU8, BU8, WB, 0, CV>), dim3((unsigned)tiles), dim3(kThreads),
+  const int64_t tiles = ((p.M + 64 * MB - 1) / (64 * MB)) * ((p.N + kBN - 1) / kBN) * p.batch;
+  hipLaunchKernelGGL((MfmaGemmKernel<KIND, OUT, ZP, AU8, BU8, WB, 0, CV, MB>), dim3((unsigned)tiles), dim3(kThreads),
                      0, s, p);
+}
+
+// Rounds of the chip's 256 CUs that `tiles` workgroups of the core take (one
+// per CU: each holds 72 to 144 KB of LDS).
+inline int64_t Rounds(int64_t tiles) { return (tiles + 255) / 256; }
+
+// Whether 128 x 128 tiles beat 256 x 128 ones, whose count leaves CUs idle in
+// the last round.  A round of the half tile takes 0.6 of a whole one's time
+// (0.55 with fp8 weights, which leave LDS for two workgroups per CU).  At
+// K = 4096, whole -> half: int8 1024 x 4096 (1 round either way) 27.5 -> 21.0 us,
+// 1024 x 11008 (2 and 3) 60.1 -> 55.9 us, 2048 x 4096 (1 and 2) 36.1 against
+// 40.2 us; fp8 1024 x 4096 43.5 -> 32.7 us, 256 x 14336 39.6 -> 29.4 us; fp16
+// 1024 x 4096 41.9 -> 27.9 us.
+template <int KIND> inline bool PrefersHalfTile(const GemmArgs &p) {
+  const int64_t nbn = (p.N + 127) / 128 * p.batch;
+  return (KIND == kBf16F8 ? 11 : 12) * Rounds((p.M + 127) / 128 * nbn) < 20 * Rounds((p.M + 255) / 256 * nbn);
 }
 
 // Eligibility with B given transposed ([N, K] row-major, GM == 3): K a
@@ -1011,9 +1035,9 @@ inline bool EligibleBT(const GemmArgs &p) {
          p.M * p.N * 2 < lim;
 }
 
-template <int OUT> inline void LaunchBT(const GemmArgs &p, hipStream_t s) {
-  const int64_t tiles = ((p.M + kBM - 1) / kBM) * ((p.N + 127) / 128);
-  hipLaunchKernelGGL((MfmaGemmKernel<kH16, OUT, false, false, false, 2, 3>), dim3((unsigned)tiles), dim3(kThreads), 0,
+template <int OUT, int MB = 4> inline void LaunchBT(const GemmArgs &p, hipStream_t s) {
+  const int64_t tiles = ((p.M + 64 * MB - 1) / (64 * MB)) * ((p.N + 127) / 128);
+  hipLaunchKernelGGL((MfmaGemmKernel<kH16, OUT, false, false, false, 2, 3, false, MB>), dim3((unsigned)tiles), dim3(kThreads), 0,
                      s, p);
 }
 
@@ -1021,9 +1045,9 @@ template <int OUT> inline void LaunchBT(const GemmArgs &p, hipStream_t s) {
 // routing table holds (the rest leave at once).
 // WB = 4 (256-column tiles, fp8 B only) needs K % kKStep == 0 and routing
 // tables counted in 256-column tiles.
-template <int OUT, int GM, int KIND = kH16, int WB = 2>
+template <int OUT, int GM, int KIND = kH16, int WB = 2, int MB = 4>
 inline void LaunchGrouped(const GemmArgs &p, int64_t max_tiles, hipStream_t s) {
-  hipLaunchKernelGGL((MfmaGemmKernel<KIND, OUT, false, false, false, WB, GM>), dim3((unsigned)max_tiles),
+  hipLaunchKernelGGL((MfmaGemmKernel<KIND, OUT, false, false, false, WB, GM, false, MB>), dim3((unsigned)max_tiles),
                      dim3(kThreads), 0, s, p);
 }
 

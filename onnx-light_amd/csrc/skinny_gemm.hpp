@@ -398,13 +398,15 @@ inline bool PrefersSkinny(const mg::GemmArgs &p, bool i8, bool zp) {
   return rows <= 32 && p.K >= 2048 && (p.N + 63) / 64 * p.batch <= (i8 ? 64 : 256);
 }
 
-// Whether a grouped call goes here instead of the routed 256-row core, whose
-// tiles are nearly empty then: by the average number of pairs per expert and
-// the columns of all experts.  bf16 x fp8 experts, K = 4096: 8 x N = 14336 with
-// 2 / 8 / 16 / 32 pairs per expert 91 / 101 / 115 / 176 against 158 / 161 / 167 /
-// 171 us; 8 x N = 1024 with 16 / 64 pairs 18.6 / 46 against 79 / 81 us.
+// Whether a grouped call goes here instead of the routed core, whose tiles are
+// nearly empty then: by the average number of pairs per expert and the columns
+// of all experts.  bf16 x fp8 experts, K = 4096, here against the core's 128-row
+// tiles: 8 x N = 14336 with 8 / 16 / 32 pairs per expert 101 / 117 / 178 against
+// 107 / 114 / 120 us; 8 x N = 4096 with 16 / 32 pairs 25.8 / 41.5 against 33.1 / 33.8
+// us; 8 x N = 1024 with 32 / 64 pairs 29.8 / 46.4 against 31.5 / 32.7 us.
 inline bool PrefersSkinnyGrouped(const mg::GemmArgs &p) {
-  const int64_t pairs = p.M * p.grp_sel, most = p.grp_count * p.N <= 40960 ? 64 : 32;
+  const int64_t pairs = p.M * p.grp_sel, cols = p.grp_count * p.N;
+  const int64_t most = cols <= 16384 ? 32 : (cols <= 65536 ? 16 : 12);
   return pairs <= kMaxPairs && pairs <= most * p.grp_count && p.N >= 64 && p.N <= (int64_t(1) << 26) && p.K >= 32;
 }
 

@@ -514,15 +514,15 @@ inline int64_t Tiles(const GemmArgs &p, int side) {
   return (p.M + side - 1) / side * ((p.N + side - 1) / side) * p.batch;
 }
 
-// Whether p goes to 64 x 64 tiles: up to two of them per CU.  The core's
-// 256 x 128 tiles then leave most CUs idle (at K = 4096, int8 / fp8 / fp16:
-// 256 x 4096 outputs are 32 core tiles or 256 small ones, 25.5 -> 14.3 us /
-// 41.9 -> 26.0 us / 38.2 -> 23.7 us; 512 x 4096, 512 small tiles, 26.0 -> 21.2 /
-// 43.5 -> 37.7 / 39.1 -> 34.3 us).  Past that the small tile's LDS traffic per
-// product loses (1024 x 4096, 1024 small tiles: 28.1 against 39.4 us int8,
-// 41.9 against 67.1 us fp16); the shapes the core does not take then run in
-// 128 x 128 tiles (30.0 and 51.0 us there; at 688 small tiles the two tie).
-inline bool PrefersSmallTile(const GemmArgs &p) { return Tiles(p, 64) <= 512; }
+// Whether p goes to 64 x 64 tiles.  Where the core takes p as well (`core`), up
+// to one of them per CU: at K = 4096, int8 / fp8 / fp16, 256 x 4096 outputs (256
+// small tiles) take 14.1 / 24.0 / 23.7 us here and 15.5 / 25.6 / 24.2 us in the
+// core's 128 x 128 tiles; 512 x 4096 (512 small tiles) 21.4 / 35.4 / 34.3 against
+// 16.7 / 26.6 / 25.6 us, the small tile's LDS traffic per product being twice the
+// core's.  The shapes the core does not take go on to two per CU, then to
+// 128 x 128 tiles of this kernel (1024 x 4096: 39.4 -> 30.0 us int8, 67.1 -> 51.0 us
+// fp16; at 688 small tiles the two tie).
+inline bool PrefersSmallTile(const GemmArgs &p, bool core) { return Tiles(p, 64) <= (core ? 256 : 512); }
 
 template <int KIND, int SRC, int OUT, bool ZP> inline void Launch(const GemmArgs &p, bool big, hipStream_t s) {
   if (big)

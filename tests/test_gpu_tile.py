@@ -90,3 +90,34 @@ def test_b_transposed(olamd, dev, M, N, K):
     y = olamd.dequantize_packed_matmul(a.to(torch.float16), x, "gguf:q8_0", (N, K))
     exact = a.double() @ (q.double().view(N, K) * 0.5).t().contiguous()
     assert torch.equal(y, exact.to(torch.float32).to(torch.float16))
+
+
+# The core's 128-row tiles: enough outputs for them, rows that end inside one,
+# half a K step at the end.
+@pytest.mark.parametrize("M,K,N", [(520, 192, 2064), (1100, 64, 1040), (385, 320, 2176)], ids=str)
+def test_half_tiles(olamd, dev, M, K, N):
+    g = torch.Generator(device=dev).manual_seed(M)
+    ints = lambda lo, hi, sh: torch.randint(lo, hi, sh, generator=g, device=dev, dtype=torch.int32)  # noqa: E731
+    for lo_a, dt_a, lo_b, dt_b in ((0, torch.uint8, -128, torch.int8), (-128, torch.int8, 0, torch.uint8)):
+        a, b = ints(lo_a, lo_a + 256, (M, K)).to(dt_a), ints(lo_b, lo_b + 256, (K, N)).to(dt_b)
+        za, zb = ints(lo_a, lo_a + 256, (M,)).to(dt_a), ints(lo_b, lo_b + 256, (N,)).to(dt_b)
+        y = olamd.matmul_integer(a, b, za, zb)
+        assert torch.equal(y.double(), (a.double() - za.double().unsqueeze(1)) @ (b.double() - zb.double()))
+        assert torch.equal(olamd.matmul_integer(a, b).double(), a.double() @ b.double())
+    a, b = ints(-2, 3, (M, K)), ints(-8, 9, (K, N))
+    exact = a.double() @ b.double()
+    for dt in (torch.float16, torch.bfloat16):
+        assert torch.equal(olamd.matmul(a.to(dt), b.to(dt)), exact.to(torch.float32).to(dt))
+    scale = torch.pow(2.0, -ints(0, 4, (N,)).float())
+    w = b.to(torch.float32).to(torch.float8_e4m3fn)
+    y = olamd.dequantize_linear_matmul(a.to(torch.bfloat16), w, scale, None, 1, olamd.BFLOAT16)
+    assert torch.equal(y, (exact * scale.double()).to(torch.float32).to(torch.bfloat16))
+    # grouped: 16-bit experts given [N, K], and fp8 experts [K, N]
+    idx = ints(0, 2, (M, 1))
+    e = torch.stack((b, -b)).to(torch.float32)
+    want = torch.where(idx.unsqueeze(2) == 0, exact.unsqueeze(1), -exact.unsqueeze(1))
+    y = olamd.grouped_matmul(a.to(torch.bfloat16), e.transpose(1, 2).contiguous().to(torch.bfloat16), idx, transB=1)
+    assert torch.equal(y, want.to(torch.float32).to(torch.bfloat16))
+    y = olamd.dequantize_linear_grouped_matmul(a.to(torch.bfloat16), e.to(torch.float8_e4m3fn),
+                                               torch.ones((2, 1, N), device=dev), idx, cast_to=olamd.BFLOAT16)
+    assert torch.equal(y, want.to(torch.float32).to(torch.bfloat16))
