@@ -1522,6 +1522,16 @@ int DqMatMul(const onnxl_amd_tensor *a, const onnxl_amd_tensor *x, const onnxl_a
              hipStream_t stream) {
   DqMatMulParams p = PlanDqMatMul(a, x, x_scale, x_zp, axis, cast_to, y);
   const bool has_zp = !Absent(x_zp);
+  // The kernel, and with it the scratch, depends on the device addresses'
+  // alignment: staged host payloads sit in 256-byte aligned scratch.
+  auto addr = [](const onnxl_amd_tensor *t) -> void * {
+    return t->location == ONNXL_AMD_HOST ? reinterpret_cast<void *>(uintptr_t(256)) : t->data;
+  };
+  p.A = addr(a);
+  p.W = static_cast<const uint8_t *>(addr(x));
+  p.scale = addr(x_scale);
+  p.zp = has_zp ? static_cast<const uint8_t *>(addr(x_zp)) : nullptr;
+  p.Y = addr(y);
   const size_t scratch_bytes = DqMatMulScratchBytes(p);
   Staging st(stream, scratch_bytes, {a, x, x_scale, has_zp ? x_zp : nullptr}, {y});
   p.A = st.In(a);
@@ -1553,7 +1563,7 @@ int DqMatMulNoAlloc(const onnxl_amd_tensor *a, const onnxl_amd_tensor *x, const 
   p.scale = x_scale->data;
   p.zp = has_zp ? static_cast<const uint8_t *>(x_zp->data) : nullptr;
   p.Y = y->data;
-  const size_t need = DqMatMulScratchBytes(p), nc = DqMatMulCounters(p);
+  const size_t need = DqMatMulFixedScratchBytes(p), nc = DqMatMulCounters(p);
   if (need > kNoAllocDataBytes || nc * sizeof(unsigned) > kNoAllocCounterBytes)
     throw Unsupported(Cat(kDqmName, ": this call needs ", need, " bytes of scratch and ", nc,
                           " counters; the no-allocation entry point holds ", kNoAllocDataBytes, " bytes and ",

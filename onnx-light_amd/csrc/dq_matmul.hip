@@ -2,13 +2,17 @@
 //
 //  - int4 / uint4 weights with FLOAT16 scales, M <= 16 (decode): the
 //    bandwidth-bound GEMV, on the ONNX packing (gemv_q4.hip) or on the tiled
-//    layout of a prepared weight (gemv_q4_tiled.hip).
+//    layout of a prepared weight (gemv_q4_tiled.hip, also more rows in slabs).
+//  - prepared int4 / uint4 weights, FLOAT16 activations and scales, more rows:
+//    the pipelined MFMA core with the weight decoded as its fragments are read
+//    from LDS (mfma_gemm.hpp, kF16I4).
 //  - float8e4m3fn weights, FLOAT scales per column or per tensor, Cast to
 //    BFLOAT16, bf16 activations (prefill): the pipelined MFMA core with the
 //    weight decoded exactly to bf16 as it is read from LDS and the scale
 //    applied to the fp32 sums (mfma_gemm.hpp, kBf16F8); the decode GEMM
-//    (skinny_gemm.hpp) for a few rows; the small-tile GEMM for few outputs, and for the shapes and alignments the core does not
-//    take, there with each weight rounded as the chain rounds it.
+//    (skinny_gemm.hpp) for a few rows; the small-tile GEMM for few outputs, and
+//    for the shapes and alignments the core does not take, there with each
+//    weight rounded as the chain rounds it.
 //  - anything else the C ABI accepts: the weight is dequantised into scratch
 //    with the chain's exact rounding, then multiplied by the 16-bit MatMul.
 #include <algorithm>
@@ -168,6 +172,47 @@ mg::GemmArgs Fp8Args(const DqMatMulParams &p) {
   return g;
 }
 
+// Prepared 4-bit weights past the GEMV's rows, decoded inside the GEMM: fp16
+// activations and scales, one scale row per 32 or more rows of k (a power of
+// two) or one for all.  Dequantising the whole weight first costs a pass over
+// it and over its fp16 form for every call (K = 4096, N = 11008: 20 us if it
+// ran at the copy rate, 128 us as it was), more than the decode adds to the
+// GEMM (M = 1000: fp16 weight 94 us, this 104 us).
+mg::GemmArgs Int4Args(const DqMatMulParams &p) {
+  mg::GemmArgs g{};
+  g.A = p.A;
+  g.B = p.W;
+  g.Y = p.Y;
+  g.M = p.M;
+  g.N = p.N;
+  g.K = p.K;
+  g.batch = 1;
+  g.scale = p.scale;
+  g.scale_rows = p.mode == 2 ? p.K / p.block : 1;
+  g.blk_shift = p.mode == 2 ? __builtin_ctzll((unsigned long long)p.block) : 31;
+  g.zp4 = p.zp;
+  g.w_signed = p.w_dtype == kInt4;
+  return g;
+}
+
+bool Int4GemmEligible(const DqMatMulParams &p) {
+  if (!p.w_tiled || p.a_bf16 || !p.scale_f16 || !p.deq_round_f16 || p.cast_round != 0) return false;
+  if (p.mode == 2 ? p.block < 32 || (p.block & (p.block - 1)) != 0 : p.mode != 1) return false;
+  return mg::EligibleI4(Int4Args(p));
+}
+
+void LaunchInt4Gemm(const DqMatMulParams &p, hipStream_t stream) {
+  const mg::GemmArgs g = Int4Args(p);
+  const bool half = mg::PrefersHalfTile<mg::kF16I4>(g);
+  if (p.zp != nullptr) {
+    if (half) mg::Launch<mg::kF16I4, mg::kOutF16, true, false, false, 2, false, 2>(g, stream);
+    else mg::Launch<mg::kF16I4, mg::kOutF16, true, false, false>(g, stream);
+  } else {
+    if (half) mg::Launch<mg::kF16I4, mg::kOutF16, false, false, false, 2, false, 2>(g, stream);
+    else mg::Launch<mg::kF16I4, mg::kOutF16, false, false, false>(g, stream);
+  }
+}
+
 }  // namespace
 
 void LaunchHMatMul(const HMatMulParams &p, hipStream_t stream) {
@@ -198,7 +243,16 @@ void LaunchHMatMulBT(const HMatMulParams &p, hipStream_t stream) {
 }
 
 size_t DqMatMulScratchBytes(const DqMatMulParams &p) {
-  if (GemvQ4TiledEligible(p)) return 0;
+  if (GemvQ4TiledEligible(p) || Int4GemmEligible(p) || Fp8Eligible(p)) return 0;
+  if (GemvQ4Eligible(p)) return GemvQ4ScratchBytes(p);
+  return (size_t)(p.K * p.N) * sizeof(uint16_t);
+}
+
+// The scratch that bounds the no-allocation entry point: a call whose weight
+// would not fit there dequantised is refused, also where the kernel that
+// takes it needs none.
+size_t DqMatMulFixedScratchBytes(const DqMatMulParams &p) {
+  if (p.M <= 16 && GemvQ4TiledEligible(p)) return 0;
   if (GemvQ4Eligible(p)) return GemvQ4ScratchBytes(p);
   if (Fp8Eligible(p) && mg::Eligible<mg::kBf16F8>(Fp8Args(p))) return 0;
   return (size_t)(p.K * p.N) * sizeof(uint16_t);
@@ -218,6 +272,10 @@ bool LaunchDqMatMul(const DqMatMulParams &p, void *scratch, size_t scratch_bytes
   if (GemvQ4Eligible(p)) {
     if (scratch_bytes < GemvQ4ScratchBytes(p) || n_counters < GemvQ4Counters(p)) return false;
     LaunchGemvQ4(p, scratch, counters, stream);
+    return true;
+  }
+  if (Int4GemmEligible(p)) {
+    LaunchInt4Gemm(p, stream);
     return true;
   }
   if (Fp8Eligible(p)) {

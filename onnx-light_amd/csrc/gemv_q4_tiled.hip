@@ -29,6 +29,8 @@
 //    the exact integer x - zp, and one packed fp16 multiply by the scale
 //    rounds fp16(float(x - zp) * scale) (the fp32 product of a 5-bit integer
 //    and an fp16 scale is exact);
+//  - more rows than 16 run as slabs of 32, two MFMAs per decoded fragment
+//    (PrefersGemv draws the line to the 4-bit GEMM);
 //  - the waves' fp32 partial sums are reduced through LDS in a fixed order
 //    and stored as fp16 (round to nearest even).
 #include <algorithm>
@@ -36,6 +38,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "mfma_gemm.hpp"
 
 namespace onnxl_amd {
 namespace {
@@ -53,6 +56,7 @@ constexpr int kGroupBytes = 1024;
 constexpr int kDepth = 2;            // row groups whose loads are in flight ahead of use
 constexpr int kMaxTiles = 4;         // tiles per workgroup
 constexpr int kTargetGroups = 256;   // workgroups wanted: one per CU
+constexpr int kSlabRows = 32;        // activation rows per workgroup past 16
 
 constexpr int kRsrcWord3 = 0x00020000;
 constexpr unsigned kOob = 0x80000000u;  // past every buffer: loads return zero, stores drop
@@ -96,15 +100,19 @@ __device__ __forceinline__ uint32_t OddBias(uint32_t b) { return 0x5400u + ((b -
 
 // MODE: 0 per-tensor, 1 per-column, 2 blocked along K, 3 blocked with blocks
 // of 128 rows or more (one scale row per 128-row group, loaded once).
-template <int T, bool HAS_ZP, bool SIGNED, int MODE>
+// MT: sets of 16 activation rows (a workgroup's slab is the 16 * MT rows from
+// 16 * MT * blockIdx.y); a decoded weight fragment feeds all of them.
+template <int T, bool HAS_ZP, bool SIGNED, int MODE, int MT>
 __global__ __launch_bounds__(kThreads) void GemvQ4TiledKernel(const TiledArgs p) {
   constexpr bool kBlocked = MODE >= 2;
   constexpr int kPitch = 16 * T + 4;  // floats per activation row of a wave's partial sums
-  __shared__ __attribute__((aligned(16))) float red[kWaves][16][kPitch];
+  __shared__ __attribute__((aligned(16))) float red[kWaves][16 * MT][kPitch];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
   const int li = lane & 15, g = lane >> 4;
   const int tile0 = blockIdx.x * T;
+  const int row0 = 16 * MT * (int)blockIdx.y;
+  const int M = min(p.M - row0, 16 * MT);  // rows of this slab
   // this wave's 128-row groups [gb, gb + ng)
   const int gb = wave * p.ngroups / kWaves;
   const int ng = (wave + 1) * p.ngroups / kWaves - gb;
@@ -112,7 +120,7 @@ __global__ __launch_bounds__(kThreads) void GemvQ4TiledKernel(const TiledArgs p)
   const int64_t s_rows = kBlocked ? p.K >> p.blk_shift : 1;
 
   const __amdgpu_buffer_rsrc_t rsW = Rsrc(p.W, p.ntiles * tile_bytes);
-  const __amdgpu_buffer_rsrc_t rsA = Rsrc(p.A, (int64_t)p.M * p.K * 2);
+  const __amdgpu_buffer_rsrc_t rsA = Rsrc(p.A + (int64_t)row0 * p.K, (int64_t)M * p.K * 2);
   const __amdgpu_buffer_rsrc_t rsS = Rsrc(p.scale, kBlocked ? s_rows * p.N * 2 : (MODE == 1 ? p.N * 2 : 2));
   const __amdgpu_buffer_rsrc_t rsZ =
       Rsrc(p.zp, HAS_ZP ? (kBlocked ? (s_rows * p.N + 1) / 2 : (MODE == 1 ? (p.N + 1) / 2 : 1)) : 0);
@@ -151,12 +159,14 @@ __global__ __launch_bounds__(kThreads) void GemvQ4TiledKernel(const TiledArgs p)
   // ---- one slot per row group in flight: weights, activations, and (mode 2)
   // the scale / zero point of each chunk ----
   v4i wq[kDepth][T];
-  v8h act[kDepth][4];
+  v8h act[kDepth][4][MT];
   uint32_t sc[kDepth][T][4];
   uint32_t zq[kDepth][T][4];
-  v4f acc[T];
+  v4f acc[MT][T];
 #pragma unroll
-  for (int t = 0; t < T; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < T; ++t) acc[m][t] = v4f{0.f, 0.f, 0.f, 0.f};
 
   // Row group i of this wave into slot s.  Every offset is a per-lane
   // constant (vector offset) plus a wave-uniform part (scalar offset), so the
@@ -164,8 +174,10 @@ __global__ __launch_bounds__(kThreads) void GemvQ4TiledKernel(const TiledArgs p)
   // past M and rows past K read zero activations (a vector offset past the
   // buffer); the weights there are padding or zeros and the scale row is
   // clamped into the scale tensor, so those products are exactly 0.
-  const bool m_ok = li < p.M;
-  const unsigned a_lane = m_ok ? ((unsigned)(li * p.K) * 2u + 16u * (unsigned)g) : kOob;  // bytes
+  unsigned a_lane[MT];  // bytes
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+    a_lane[m] = 16 * m + li < M ? (unsigned)((16 * m + li) * p.K) * 2u + 16u * (unsigned)g : kOob;
   // K % 32 == 0: a 32-row chunk lies wholly inside or wholly past K.  The
   // scale row of lane g is (rb >> shift) + g_srow; clamping the uniform part
   // to s_rows - 1 - (24 >> shift) keeps every lane inside the scale tensor and
@@ -189,8 +201,10 @@ __global__ __launch_bounds__(kThreads) void GemvQ4TiledKernel(const TiledArgs p)
     for (int c = 0; c < 4; ++c) {
       const int rb = q * kGroupRows + 32 * c;  // first row of chunk c (wave-uniform)
       const bool in_k = live && rb < p.K;      // wave-uniform
-      act[s][c] = __builtin_bit_cast(
-          v8h, __builtin_amdgcn_raw_buffer_load_b128(rsA, in_k ? a_lane : kOob, in_k ? 2 * rb : 0, 0));
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        act[s][c][m] = __builtin_bit_cast(
+            v8h, __builtin_amdgcn_raw_buffer_load_b128(rsA, in_k ? a_lane[m] : kOob, in_k ? 2 * rb : 0, 0));
       if constexpr (kBlocked) {
         const int su = min(rb >> p.blk_shift, su_max);  // wave-uniform
 #pragma unroll
@@ -235,7 +249,9 @@ __global__ __launch_bounds__(kThreads) void GemvQ4TiledKernel(const TiledArgs p)
           wop[2 * j] = v.x;
           wop[2 * j + 1] = v.y;
         }
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wop, act[s][c], acc[t], 0, 0, 0);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wop, act[s][c][m], acc[m][t], 0, 0, 0);
       }
     }
   };
@@ -259,15 +275,17 @@ __global__ __launch_bounds__(kThreads) void GemvQ4TiledKernel(const TiledArgs p)
   // move on
   __builtin_amdgcn_s_waitcnt(0);
 
-  // ---- reduce the waves: lane (li, g), register q of acc[t] holds row m = li
-  // of column 16 * (tile0 + t) + 4g + q ----
-  const int M = p.M;
-  if (li < M) {
+  // ---- reduce the waves: lane (li, g), register q of acc[m][t] holds row
+  // 16 m + li of column 16 * (tile0 + t) + 4g + q ----
 #pragma unroll
-    for (int t = 0; t < T; ++t) *reinterpret_cast<v4f *>(&red[wave][li][16 * t + 4 * g]) = acc[t];
+  for (int m = 0; m < MT; ++m) {
+    if (16 * m + li < M) {
+#pragma unroll
+      for (int t = 0; t < T; ++t) *reinterpret_cast<v4f *>(&red[wave][16 * m + li][16 * t + 4 * g]) = acc[m][t];
+    }
   }
   __syncthreads();
-  const __amdgpu_buffer_rsrc_t rsY = Rsrc(p.Y, (int64_t)M * p.N * 2);
+  const __amdgpu_buffer_rsrc_t rsY = Rsrc(p.Y + (int64_t)row0 * p.N, (int64_t)M * p.N * 2);
   const int col0 = 16 * tile0;
   for (int j = threadIdx.x; j < M * 4 * T; j += kThreads) {
     const int m = j / (4 * T), cq = 4 * (j % (4 * T));
@@ -322,6 +340,25 @@ int TilesPerGroup(int64_t ntiles) {
   return (int)std::min<int64_t>(kMaxTiles, std::max<int64_t>(1, (ntiles + kTargetGroups - 1) / kTargetGroups));
 }
 
+// Rows that this kernel takes: 16, and past them slabs of 32 while those cost
+// less than the 4-bit GEMM's tiles (mfma_gemm.hpp).  A round of 256 workgroups
+// with T tiles each takes about 5 + T units, one of the GEMM's 128-row tiles
+// 22 and of its 256-row tiles 40.  Slabs against the GEMM at K = 4096: N =
+// 11008 (T = 3) 32 rows 12.6 / 34.7 us, 64 rows 23.6 / 35.0, 96 rows 33.8 /
+// 35.4, 128 rows 44.0 / 35.6; N = 4096 (T = 1) 96 rows 26.5 / 34.6, 128 rows
+// 34.2 / 34.5; N = 1024 (4 slabs to a round) 128 rows 10.5 / 34.6, 256 rows
+// 18.5 / 34.4.  At K = 1024: N = 11008 64 rows 9.0 / 11.9, 96 rows 12.6 / 11.9;
+// N = 4096 96 rows 9.8 / 11.8, 128 rows 12.2 / 11.8.  Slabs of 16 rows decode
+// every weight twice as often (N = 11008 64 rows 28.9 us); slabs of 64 gain
+// only where they are full (20.9 us; 48 rows of N = 1024 14.9 against 10.1).
+bool PrefersGemv(int64_t M, int64_t N, int64_t K) {
+  if (M <= 16) return M >= 1;
+  if (K == 0) return false;
+  const int64_t ntiles = (N + 15) / 16, nbn = (N + 127) / 128, T = TilesPerGroup(ntiles);
+  const int64_t rounds = mg::Rounds((ntiles + T - 1) / T * ((M + kSlabRows - 1) / kSlabRows));
+  return (5 + T) * rounds <= std::min(22 * mg::Rounds((M + 127) / 128 * nbn), 40 * mg::Rounds((M + 255) / 256 * nbn));
+}
+
 }  // namespace
 
 int64_t TiledInt4Bytes(int64_t K, int64_t N) {
@@ -339,7 +376,7 @@ void LaunchTileInt4(const uint8_t *x, int64_t K, int64_t N, int is_signed, uint3
 bool GemvQ4TiledEligible(const DqMatMulParams &p) {
   const bool four = p.w_dtype == kInt4 || p.w_dtype == kUint4;
   const int64_t lim = (int64_t(1) << 31) - 64;
-  return p.w_tiled && four && p.M >= 1 && p.M <= 16 && !p.a_bf16 && p.scale_f16 && p.deq_round_f16 &&
+  return p.w_tiled && four && PrefersGemv(p.M, p.N, p.K) && !p.a_bf16 && p.scale_f16 && p.deq_round_f16 &&
          p.cast_round == 0 && p.K % 32 == 0 &&
          (p.mode != 2 || (p.block >= 8 && (p.block & (p.block - 1)) == 0)) &&
          (p.zp == nullptr || p.N % 2 == 0) && TiledInt4Bytes(p.K, p.N) < lim && p.M * p.K * 2 < lim &&
@@ -364,7 +401,8 @@ void LaunchGemvQ4Tiled(const DqMatMulParams &p, hipStream_t stream) {
   const uint32_t b = 0x6400u + (sgn ? 8u : 0u);
   g.bias2 = b | (b << 16);
   const int T = TilesPerGroup(g.ntiles);
-  const dim3 grid((unsigned)((g.ntiles + T - 1) / T));
+  const int rows = p.M <= 16 ? 16 : kSlabRows;
+  const dim3 grid((unsigned)((g.ntiles + T - 1) / T), (unsigned)((g.M + rows - 1) / rows));
   const bool zp = p.zp != nullptr;
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, stream, g); };
   auto by_mode = [&](auto k0, auto k1, auto k2, auto k3) {
@@ -373,21 +411,25 @@ void LaunchGemvQ4Tiled(const DqMatMulParams &p, hipStream_t stream) {
     else if (g.blk_shift < 7) go(k2);
     else go(k3);
   };
-#define OLA_TILED(TT, ZP, SG)                                                                    \
-  by_mode(GemvQ4TiledKernel<TT, ZP, SG, 0>, GemvQ4TiledKernel<TT, ZP, SG, 1>, GemvQ4TiledKernel<TT, ZP, SG, 2>, \
-          GemvQ4TiledKernel<TT, ZP, SG, 3>)
-  auto by_zp = [&](auto tag) {
-    constexpr int TT = decltype(tag)::value;
-    if (!zp) OLA_TILED(TT, false, false);
-    else if (sgn) OLA_TILED(TT, true, true);
-    else OLA_TILED(TT, true, false);
+#define OLA_TILED(TT, ZP, SG, MM)                                                                       \
+  by_mode(GemvQ4TiledKernel<TT, ZP, SG, 0, MM>, GemvQ4TiledKernel<TT, ZP, SG, 1, MM>, GemvQ4TiledKernel<TT, ZP, SG, 2, MM>, \
+          GemvQ4TiledKernel<TT, ZP, SG, 3, MM>)
+  auto by_zp = [&](auto tag, auto rows) {
+    constexpr int TT = decltype(tag)::value, MM = decltype(rows)::value;
+    if (!zp) OLA_TILED(TT, false, false, MM);
+    else if (sgn) OLA_TILED(TT, true, true, MM);
+    else OLA_TILED(TT, true, false, MM);
   };
-  switch (T) {
-  case 1: by_zp(std::integral_constant<int, 1>{}); break;
-  case 2: by_zp(std::integral_constant<int, 2>{}); break;
-  case 3: by_zp(std::integral_constant<int, 3>{}); break;
-  default: by_zp(std::integral_constant<int, 4>{}); break;
-  }
+  auto by_t = [&](auto rows) {
+    switch (T) {
+    case 1: by_zp(std::integral_constant<int, 1>{}, rows); break;
+    case 2: by_zp(std::integral_constant<int, 2>{}, rows); break;
+    case 3: by_zp(std::integral_constant<int, 3>{}, rows); break;
+    default: by_zp(std::integral_constant<int, 4>{}, rows); break;
+    }
+  };
+  if (rows == 16) by_t(std::integral_constant<int, 1>{});
+  else by_t(std::integral_constant<int, 2>{});
 #undef OLA_TILED
 }
 

@@ -424,6 +424,7 @@ void LaunchTileInt4(const uint8_t *x, int64_t K, int64_t N, int is_signed, uint3
 bool LaunchDqMatMul(const DqMatMulParams &p, void *scratch, size_t scratch_bytes,
                     unsigned *counters, size_t n_counters, hipStream_t stream);
 size_t DqMatMulScratchBytes(const DqMatMulParams &p);
+size_t DqMatMulFixedScratchBytes(const DqMatMulParams &p);
 size_t DqMatMulCounters(const DqMatMulParams &p);
 
 // Plain FLOAT16 / BFLOAT16 MatMul (fp32 accumulate).

@@ -88,7 +88,19 @@ constexpr int kStoreThrough = 16;
 //           each s_n * q to bf16 first; the two differ by at most half a bf16
 //           ulp of each product.
 //  kH16:    fp16 x fp16 or bf16 x bf16 -> fp32 accumulate.
-enum Kind : int { kI8 = 0, kBf16F8 = 1, kH16 = 2 };
+//  kF16I4:  fp16 A x 4-bit B in the tiled layout (kernels.hpp) with fp16 scales
+//           per block of k or per column and optional zero points (ZP): each
+//           weight enters the MFMA as fp16((q - zp) * scale), the rounding of
+//           the DequantizeLinear -> MatMul chain.  A K step brings 16 KB of A,
+//           4 KB of codes (dword direct loads: the layout's 16 bytes are four
+//           k ranges) and its one or two scale rows through the ring.  Bound
+//           by the decode's VALU work beside the MFMAs (per step and wave 118
+//           instructions of 4 cycles, 16 of 32); with the decode left out
+//           1000 x 4096 x 11008 takes 90 us in place of 104 (fp16 weights 94).
+//           Codes, scales and zero points have register sets of their own:
+//           as parts of a 16-byte set the compiler moved them behind a wait
+//           for the newest LDS read (37.4 -> 34.6 us for one round of K = 4096).
+enum Kind : int { kI8 = 0, kBf16F8 = 1, kH16 = 2, kF16I4 = 3 };
 
 // Output conversions.
 // kOutQ8Row: the 8-bit requantization of kOutQ8 with a scale and an int32
@@ -114,13 +126,23 @@ template <> struct Traits<kH16> {
   static constexpr int kBsz = 2;
   using Acc = v16f;
 };
+template <> struct Traits<kF16I4> {
+  static constexpr int kKStep = 64;
+  static constexpr int kBRows = 64;
+  static constexpr int kBsz = 1;  // the layout has addresses of its own
+  using Acc = v16f;
+};
 // The workgroup tile is 256 x BN with BN = 64 * WB: each wave owns 4 x WB
 // blocks of 32 x 32 (WB = 2: 128 x 64 per wave; WB = 4: 128 x 128, which
 // halves the operand bytes per MFMA and fills the 256 accumulator registers).
 template <int KIND, int WB> constexpr int BPitch() { return 64 * WB * Traits<KIND>::kBsz; }
-template <int KIND, int WB> constexpr int BStageBytes() { return Traits<KIND>::kBRows * BPitch<KIND, WB>(); }
-// direct loads of B per wave per K step, 1 KB per instruction
-template <int KIND, int WB> constexpr int BLoadsPerWave() { return BStageBytes<KIND, WB>() / 1024 / 4; }
+template <int KIND, int WB> constexpr int BStageBytes() {
+  return Traits<KIND>::kBRows * BPitch<KIND, WB>() / (KIND == kF16I4 ? 2 : 1);
+}
+// direct loads of B per wave per K step, 1 KB per instruction (kF16I4: 256 bytes)
+template <int KIND, int WB> constexpr int BLoadsPerWave() {
+  return BStageBytes<KIND, WB>() / (KIND == kF16I4 ? 256 : 1024) / 4;
+}
 
 __device__ __forceinline__ int64_t MinI64(int64_t a, int64_t b) { return a < b ? a : b; }
 
@@ -154,6 +176,27 @@ __device__ __forceinline__ void DirectLoad16(__amdgpu_buffer_rsrc_t rs, const ch
   asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voffset), "s"(rs), "{m0}"(m0));
 }
 
+// The same with 4 bytes per lane.
+__device__ __forceinline__ void DirectLoad4(__amdgpu_buffer_rsrc_t rs, const char *lds, unsigned voffset) {
+  const unsigned m0 = (unsigned)(size_t)(lds_ptr_t)lds;
+  asm volatile("buffer_load_dword %0, %1, 0 offen lds" ::"v"(voffset), "s"(rs), "{m0}"(m0));
+}
+
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+// (x & mask) | magic as an fp16 pair, one instruction: the mask from a scalar
+// register, the magic from a vector one (the compiler emits two with literals).
+__device__ __forceinline__ v2h AndOr(unsigned x, unsigned mask, unsigned magic) {
+  unsigned r;
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(mask), "v"(magic));
+  return __builtin_bit_cast(v2h, r);
+}
+// Both halves of x times the low half of s, rounded to fp16.
+__device__ __forceinline__ int PkMulLow(v2h x, unsigned s) {
+  int r;
+  asm("v_pk_mul_f16 %0, %1, %2 op_sel_hi:[1,0]" : "=v"(r) : "v"(x), "v"(s));
+  return r;
+}
+
 // Waits for all but the newest `L` direct loads (the oldest in-flight ring
 // stage has then landed), retires this wave's LDS reads and joins the
 // workgroup barrier.  A __syncthreads() would wait for every load.
@@ -185,6 +228,13 @@ struct GemmArgs {
   int scale_f16;
   int scale_per_col;
   int64_t scale_grp_stride;
+  // kF16I4: `scale` holds scale_rows rows of N fp16 values, row k >> blk_shift
+  // for weight row k (blk_shift 31: one row); zp4 the packed zero points of the
+  // same shape (ZP kernels); w_signed: INT4 codes (stored offset by 8)
+  int64_t scale_rows;
+  int blk_shift;
+  const uint8_t *zp4;
+  int w_signed;
   // Row pitches of B and Y in elements (0: N), so a launch can cover a
   // column range of larger matrices; N stays the width computed.
   int64_t ldb, ldy;
@@ -231,13 +281,15 @@ __device__ __forceinline__ uint32_t DivMagic(uint32_t x, uint32_t magic) {
 // MB: 32-row blocks per wave.  4 is the 256-row tile; 2 halves it (128 rows),
 // for problems whose 256-row tiles leave CUs idle.
 template <int KIND, int OUT, bool ZP, bool AU8, bool BU8, int WB, int GM = 0, bool CV = false, int MB = 4>
-__global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void MfmaGemmKernel(const GemmArgs p) {
+__global__ __launch_bounds__(kThreads, MB == 2 && (KIND == kBf16F8 || KIND == kF16I4) ? 2 : 1) void MfmaGemmKernel(const GemmArgs p) {
   constexpr int BM = 64 * MB, AST = BM * kStepBytes;  // tile rows, bytes of an A stage
   constexpr int LA = AST / 1024 / 4;                  // direct loads of A per wave per K step
   static_assert(MB == 4 || (MB == 2 && WB == 2), "tile height");
   constexpr bool RA = ZP, CB = ZP;
   constexpr bool GRP = GM == 1 || GM == 2;  // grouped (routing tables)
   constexpr bool BT = GM == 2 || GM == 3 || CV;
+  constexpr bool I4 = KIND == kF16I4;
+  static_assert(!I4 || (WB == 2 && GM == 0), "4-bit weights: 128-column tiles");
   static_assert(GM == 0 || (((KIND == kH16 && WB == 2) || (KIND == kBf16F8 && GM == 1)) && !ZP),
                 "grouped mode: 16-bit operands in 128-column tiles, or fp8 B [K, N] per group");
   static_assert(!CV || (KIND == kI8 && WB == 2 && GM == 0), "implicit convolution: int8, 128-column tiles");
@@ -254,7 +306,7 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
   // different positions, where the plain one put them on 8 twice.
   constexpr int kBSwz = kBP >= 256 ? 2 : 1;
   constexpr int kBStage = BStageBytes<KIND, WB>();
-  constexpr int LB = BLoadsPerWave<KIND, WB>(), L = LA + LB;
+  constexpr int LB = BLoadsPerWave<KIND, WB>(), L = LA + LB + (I4 ? 1 : 0);  // 4-bit: and one of scales or zero points
   static_assert(WB == 2 || (WB == 4 && KIND != kH16), "tile width");
   constexpr int kOsz = OUT == kOutI32 ? 4 : (OUT == kOutQ8 || OUT == kOutQ8Row ? 1 : 2);
   static_assert(LB >= 1 && LB <= 4, "B direct loads per wave");
@@ -262,11 +314,13 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
   // tell a read of one stage from a direct load into another.
   __shared__ __align__(16) char sa0[AST], sa1[AST], sa2[AST];
   __shared__ __align__(16) char sb0[kBStage], sb1[kBStage], sb2[kBStage];
-  __shared__ int32_t zsum[ZP ? (kThreads / 64) * 2 * kWN : 1];  // per wave: CB and beta of its columns
+  __shared__ __align__(16) char ss0[I4 ? 1024 : 16], ss1[I4 ? 1024 : 16], ss2[I4 ? 1024 : 16];  // 4-bit: scales, zero points
+  __shared__ int32_t zsum[ZP && !I4 ? (kThreads / 64) * 2 * kWN : 1];  // per wave: CB and beta of its columns
   __shared__ __align__(16) float cscale[KIND == kBf16F8 ? (kThreads / 64) * kWN : 4];  // per wave: column scales
   // stage index -> array (indices are compile-time constants after unrolling)
   auto SA = [&](int s) __attribute__((always_inline)) -> char * { return s == 0 ? sa0 : (s == 1 ? sa1 : sa2); };
   auto SB = [&](int s) __attribute__((always_inline)) -> char * { return s == 0 ? sb0 : (s == 1 ? sb1 : sb2); };
+  auto SS = [&](int s) __attribute__((always_inline)) -> char * { return s == 0 ? ss0 : (s == 1 ? ss1 : ss2); };
 
   const int tid = threadIdx.x;
   // the wave index as a scalar: the LDS destinations of the direct loads (M0)
@@ -343,11 +397,16 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
   const __amdgpu_buffer_rsrc_t rsA =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(Ab), (short)0, (int)(M * KA), kRsrcWord3);
   const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<char *>(Bb), (short)0, (int)(CV ? p.cv.image_bytes : (BT ? N * KA : K * NB)), kRsrcWord3);
+      const_cast<char *>(Bb), (short)0, (int)(CV ? p.cv.image_bytes : I4 ? (N + 15) / 16 * ((K + 127) / 128) * 1024 : (BT ? N * KA : K * NB)), kRsrcWord3);
   // look-ahead loads past the last K step go through empty descriptors (every
   // access out of range): a scalar select instead of a per-lane one
   const __amdgpu_buffer_rsrc_t rsA0 = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(Ab), (short)0, 0, kRsrcWord3);
   const __amdgpu_buffer_rsrc_t rsB0 = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(Bb), (short)0, 0, kRsrcWord3);
+  // 4-bit: this wave's rows of scales (waves 0, 1) or zero points (2, 3), the
+  // rows of the step's first (even waves) or last 32 k
+  const __amdgpu_buffer_rsrc_t rsS = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void *>(wave < 2 ? p.scale : (const void *)p.zp4), (short)0,
+      (int)(!I4 ? 0 : wave < 2 ? p.scale_rows * N * 2 : ZP ? p.scale_rows * N / 2 : 0), kRsrcWord3);
   const int64_t YR = GRP ? M * p.grp_sel : M;  // rows of Y
   const __amdgpu_buffer_rsrc_t rsY = __builtin_amdgcn_make_buffer_rsrc(
       static_cast<char *>(p.Y) + bt * M * LDY * kOsz, (short)0, (int)(YR * LDY * kOsz), kRsrcWord3);
@@ -369,7 +428,14 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
 #pragma unroll
   for (int q = 0; q < LB; ++q) {
     const int i = wave * LB + q;  // 1 KB piece of the B stage
-    if constexpr (CV) {
+    if constexpr (I4) {
+      // 16-column tile i / 2 of this workgroup, 32-row chunk i % 2 of the step:
+      // one dword of each lane's four.  Odd tiles' lanes are swapped by halves,
+      // so that a fragment read of two tiles meets 64 different banks.
+      const int64_t tile = (col0 >> 4) + (i >> 1);
+      b_g[q] = 16 * tile < N ? (unsigned)(tile * ((K + 127) / 128) * 1024 + 16 * (lane ^ ((i & 2) << 4)) + 4 * (i & 1))
+                             : kOob;
+    } else if constexpr (CV) {
       // output position n: its input pixel for tap (0, 0) and channel chunk
       const int64_t n = col0 + 8 * i + (lane >> 3);
       const int64_t oh = n / p.cv.wo, ow = n - oh * p.cv.wo;
@@ -406,8 +472,8 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
   int b_rd[WB];
 #pragma unroll
   for (int j = 0; j < WB; ++j) {
-    if constexpr (BT) {
-      b_rd[j] = 0;  // bt_rd below
+    if constexpr (BT || I4) {
+      b_rd[j] = 0;  // bt_rd, i_rd below
     } else if constexpr (KIND == kI8) {
       const int krow = 16 * (g16 >> 1) + (s16 >> 1);
       const int col = wn * kWN + j * 32 + 16 * (g16 & 1) + 8 * (s16 & 1);
@@ -428,6 +494,15 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk)
     bt_rd[kk] = BT ? (wn * kWN + lr) * 128 + 16 * ((2 * kk + lg) ^ (lr & 7) ^ ((lr >> 3) & 1)) : 0;
+  // 4-bit: sub-step kk reads chunk kk / 2, lane group 2 (kk % 2) + lg of column
+  // 32 j + lr's tile, j two tiles (1 KB) after j - 1; the column's scale and
+  // zero point of that chunk
+  int i_rd[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+    i_rd[e] = (wn * 4 + (lr >> 4)) * 512 + 4 * ((16 * (2 * e + lg) + (lr & 15)) ^ ((lr >> 4) << 5));
+  const unsigned s_g = I4 ? (unsigned)(wave < 2 ? 2 * col0 + 4 * lane : (lane < 16 ? col0 / 2 + 4 * lane : kOob)) : 0;
+  const unsigned s_row = (unsigned)(wave < 2 ? 2 * N : N / 2);  // bytes of a scale / zero-point row
   // B rows per sub-step: 32 (int8) or 16 (16-bit k values)
   constexpr int kSubRows = KIND == kI8 ? 32 : 16;
 
@@ -475,6 +550,7 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
       kb = (unsigned)(ti * p.cv.tap_row + (tap - ti * (uint32_t)p.cv.kw) * p.cv.tap_col +
                       kStepBytes * ((uint32_t)step - tap * (uint32_t)p.cv.spt));
     }
+    if constexpr (I4) kb = (unsigned)((step >> 1) * 1024 + (step & 1) * 8);
     char *sa = SA(stage);
     char *sb = SB(stage);
     const __amdgpu_buffer_rsrc_t rsa = live ? rsA : rsA0, rsb = live ? rsB : rsB0;
@@ -485,8 +561,16 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
         DirectLoad16(rsa, sa + (LA * wave + q) * 1024, a_g[q] + ka);
 #pragma unroll
     for (int q = 0; q < LB; ++q)
-      if (LA + q >= lo && LA + q < hi)
-        DirectLoad16(rsb, sb + (wave * LB + q) * 1024, b_g[q] + kb);
+      if (LA + q >= lo && LA + q < hi) {
+        if constexpr (I4) DirectLoad4(rsb, sb + (wave * LB + q) * 256, b_g[q] + kb);
+        else DirectLoad16(rsb, sb + (wave * LB + q) * 1024, b_g[q] + kb);
+      }
+    if constexpr (I4) {
+      if (LA + LB >= lo && LA + LB < hi) {
+        const unsigned row = (unsigned)((64u * (unsigned)step + 32u * (wave & 1)) >> p.blk_shift);
+        DirectLoad4(live ? rsS : rsA0, SS(stage) + wave * 256, s_g + row * s_row);
+      }
+    }
   };
 
   // ---- fragments ----
@@ -497,11 +581,17 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
   // VALU work stalls the matrix pipe.
   v4i ra[3][MB];
   v4i rb[3][WB];  // raw B: kI8 2 x tr8; kBf16F8 1 x tr8 (.xy); kH16 2 x tr16
-  auto read = [&](int buf, const char *sa, const char *sb, int kk) __attribute__((always_inline)) {
+  int rc[3][I4 ? WB : 1], rs[3][I4 ? WB : 1], rz[3][I4 && ZP ? WB : 1];  // kF16I4: 8 codes, scale, zero point byte
+  auto read = [&](int buf, const char *sa, const char *sb, const char *ss, int kk) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < WB; ++j) {
       const char *base = sb + kk * kSubRows * kBP;
-      if constexpr (BT) {
+      if constexpr (I4) {
+        rc[buf][j] = *reinterpret_cast<const int *>(sb + i_rd[kk & 1] + (kk >> 1) * 256 + j * 1024);
+        rs[buf][j] = *reinterpret_cast<const uint16_t *>(ss + (kk >> 1) * 256 + 2 * (wn * kWN + j * 32 + lr));
+        if constexpr (ZP)
+          rz[buf][j] = *reinterpret_cast<const uint8_t *>(ss + 512 + (kk >> 1) * 256 + ((wn * kWN + j * 32 + lr) >> 1));
+      } else if constexpr (BT) {
         rb[buf][j] = *reinterpret_cast<const v4i *>(sb + bt_rd[kk] + j * 4096);
       } else if constexpr (KIND == kI8) {
         const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_t)(base + b_rd[j]));
@@ -538,7 +628,11 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
   // (x ^ 0x80 = x - 128) in place one sub-step ahead, under the MFMAs of the
   // sub-step before (right before their own MFMAs the flips cost 4% more
   // cycles).
-  v4i bop[KIND == kBf16F8 ? 2 : 1][WB];
+  v4i bop[KIND == kBf16F8 || I4 ? 2 : 1][WB];
+  const unsigned i4_m0 = 0x64006400u, i4_m1 = 0x54005400u;  // fp16 pairs 1024 (unit 1) and 64 (unit 1 / 16)
+  const unsigned i4_n = I4 && p.w_signed ? 8u : 0u;
+  const v2h i4_c0 = __builtin_bit_cast(v2h, i4_m0 | i4_n | i4_n << 16);
+  const v2h i4_c1 = __builtin_bit_cast(v2h, i4_m1 | i4_n << 4 | i4_n << 20);
   auto decode = [&](int rbuf, int bbuf) __attribute__((always_inline)) {
     if constexpr (KIND == kI8 && AU8) {
 #pragma unroll
@@ -548,6 +642,21 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
     for (int j = 0; j < WB; ++j) {
       if constexpr (KIND == kI8 && BU8) {
         rb[rbuf][j] ^= bflip;
+      } else if constexpr (I4) {
+        // 8 codes -> 8 fp16 weights (13 VALU instructions): a nibble OR-ed into
+        // fp16 1024 or 64 is that plus the code exactly, the packed subtract
+        // leaves the exact integer q - zp, the packed multiply rounds once, as
+        // the chain does
+        const unsigned u = (unsigned)rc[rbuf][j], t = u >> 8;
+        v2h c0 = i4_c0, c1 = i4_c1;
+        if constexpr (ZP) {
+          const unsigned n = (p.w_signed ? 8u : 0u) ^ (((unsigned)rz[rbuf][j] >> (4 * (lr & 1))) & 15u);
+          c0 = __builtin_bit_cast(v2h, 0x64006400u | n | n << 16);
+          c1 = __builtin_bit_cast(v2h, 0x54005400u | n << 4 | n << 20);
+        }
+        const unsigned sc = (unsigned)rs[rbuf][j];
+        bop[bbuf][j] = v4i{PkMulLow(AndOr(u, 0x000f000fu, i4_m0) - c0, sc), PkMulLow(AndOr(u, 0x00f000f0u, i4_m1) - c1, sc),
+                           PkMulLow(AndOr(t, 0x000f000fu, i4_m0) - c0, sc), PkMulLow(AndOr(t, 0x00f000f0u, i4_m1) - c1, sc)};
       } else if constexpr (KIND == kBf16F8) {
         const int x = rb[rbuf][j].x, y = rb[rbuf][j].y;
         bop[bbuf][j] = v4i{Fp8PairLo(x), Fp8PairHi(x), Fp8PairLo(y), Fp8PairHi(y)};
@@ -587,11 +696,11 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
           else bv = rb[abuf][j];
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, bv), av, acc[i][j], 0, 0, 0);
         }
-      } else {  // kH16 with FLOAT16 operands
+      } else {  // FLOAT16 operands
         const v8h av = __builtin_bit_cast(v8h, ra[abuf][i]);
 #pragma unroll
         for (int j = 0; j < WB; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, rb[abuf][j]), av,
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, I4 ? bop[bbuf][j] : rb[abuf][j]), av,
                                                              acc[i][j], 0, 0, 0);
       }
     }
@@ -599,8 +708,8 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
 
   // Instruction order inside a sub-step, pinned because the scheduler would
   // otherwise sink each LDS read next to its first use.
-  constexpr int kReads = MB + WB * (KIND == kBf16F8 ? 1 : 2);
-  constexpr int kDecodeValu = KIND == kBf16F8 ? 4 * WB : (KIND == kI8 ? (AU8 ? 4 * MB : 0) + (BU8 ? 4 * WB : 0) + (CB ? 4 * WB : 0) : 0);
+  constexpr int kReads = MB + WB * (I4 ? (ZP ? 3 : 2) : KIND == kBf16F8 ? 1 : 2);
+  constexpr int kDecodeValu = I4 ? (ZP ? 20 : 13) * WB : KIND == kBf16F8 ? 4 * WB : (KIND == kI8 ? (AU8 ? 4 * MB : 0) + (BU8 ? 4 * WB : 0) + (CB ? 4 * WB : 0) : 0);
   // A plain sub-step with `nvm` direct loads: each MFMA is preceded by its
   // share of the LDS reads two sub-steps ahead and followed by a direct load
   // and its share of the decode.  Reads issued all at once at the top of a
@@ -646,8 +755,8 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
     const int nb3 = (sb3 + 1) % 3, nb2 = (sb2 + 1) % 2, rb3 = (sb3 + 2) % 3;
     const int prv = (cur + 2) % 3;  // stage of step t - 1, being refilled with step t + 2
     if (kk != 2) {
-      if (kk < 2) read(rb3, SA(cur), SB(cur), kk + 2);
-      else read(rb3, SA(nxt), SB(nxt), kk - 2);
+      if (kk < 2) read(rb3, SA(cur), SB(cur), SS(cur), kk + 2);
+      else read(rb3, SA(nxt), SB(nxt), SS(nxt), kk - 2);
       if (kk == 3) issue(t + 3, cur, 1);
       else issue(t + 2, prv, 2 + kk);
       decode(nb3, nb2);
@@ -659,7 +768,7 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
       mma(sb3, sb2, 0, MB / 2);
       __builtin_amdgcn_sched_barrier(0);
       RingBarrier<L>();
-      read(rb3, SA(nxt), SB(nxt), 0);
+      read(rb3, SA(nxt), SB(nxt), SS(nxt), 0);
       issue(t + 3, cur, 0);  // first quarter of the refill
       decode(nb3, nb2);
       colsum(sb3);
@@ -717,8 +826,8 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
     issue(0, 0, 4);
     load_zp();
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    read(0, sa0, sb0, 0);
-    read(1, sa0, sb0, 1);
+    read(0, sa0, sb0, ss0, 0);
+    read(1, sa0, sb0, ss0, 1);
     decode(0, 0);
     decode(1, 1);
     colsum(0);  // before the zero-point exchange; the MFMAs run block by block in the epilogue
@@ -731,8 +840,8 @@ __global__ __launch_bounds__(kThreads, MB == 2 && KIND == kBf16F8 ? 2 : 1) void 
     issue(2, 2, 0);
     issue(2, 2, 1);
     RingBarrier<L + 2 * L / 4>();
-    read(0, sa0, sb0, 0);
-    read(1, sa0, sb0, 1);
+    read(0, sa0, sb0, ss0, 0);
+    read(1, sa0, sb0, ss0, 1);
     decode(0, 0);
     int t = 0;
     // 12 sub-steps per iteration: s % 3 and the stages repeat.  The last
@@ -1021,7 +1130,17 @@ inline int64_t Rounds(int64_t tiles) { return (tiles + 255) / 256; }
 // 1024 x 4096 41.9 -> 27.9 us.
 template <int KIND> inline bool PrefersHalfTile(const GemmArgs &p) {
   const int64_t nbn = (p.N + 127) / 128 * p.batch;
-  return (KIND == kBf16F8 ? 11 : 12) * Rounds((p.M + 127) / 128 * nbn) < 20 * Rounds((p.M + 255) / 256 * nbn);
+  return (KIND == kBf16F8 || KIND == kF16I4 ? 11 : 12) * Rounds((p.M + 127) / 128 * nbn) < 20 * Rounds((p.M + 255) / 256 * nbn);
+}
+
+// Eligibility of the 4-bit kernel: as Eligible, with the tiled weight and its
+// scale rows below 2^31 - 2^24 bytes and 4-byte aligned.
+inline bool EligibleI4(const GemmArgs &p) {
+  const int64_t lim = (int64_t(1) << 31) - (int64_t(1) << 24);
+  auto al = [](const void *q, int n) { return reinterpret_cast<uintptr_t>(q) % n == 0; };
+  return p.K > 0 && p.K % 32 == 0 && p.N % 16 == 0 && p.batch == 1 && al(p.A, 16) && al(p.B, 16) && al(p.Y, 16) &&
+         al(p.scale, 4) && al(p.zp4, 4) && p.M * p.K * 2 + 4 * kStepBytes < lim && p.M * p.N * 4 < lim &&
+         (p.N + 15) / 16 * ((p.K + 127) / 128 + 2) * 1024 < lim && (p.scale_rows + 8) * p.N * 2 < lim;
 }
 
 // Eligibility with B given transposed ([N, K] row-major, GM == 3): K a

@@ -1,0 +1,54 @@
+"""Prepared 4-bit weights past 16 rows: the GEMV's 32-row slabs and the GEMM that
+decodes its operand (128- and 256-row tiles), at partial slabs, tiles and K
+steps, every block size, both types, with and without zero points, and operands
+that only the general path takes.  Small integers and power-of-two scales, whose
+sums are exact in any order, against 64-bit products; one-hot rows with random
+scales, which give the dequantised weights themselves, bit for bit against the
+general path on the ONNX packing."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev(olamd):
+    olamd.init(0)
+    return torch.device("cuda:0")
+
+
+# rows 17 to 96 are slabs at these sizes, the rest the GEMM
+@pytest.mark.parametrize("M,K,N", [(17, 128, 16), (33, 96, 77), (64, 384, 4112), (97, 256, 8208), (257, 32, 8208),
+                                   (129, 416, 11024), (1500, 224, 2064), (2049, 160, 2176)], ids=str)
+@pytest.mark.parametrize("block", [8, 32, 64, 128, 0, -1])  # 0: a scale per column, -1: one scale
+def test_prepared_rows(olamd, dev, M, K, N, block):
+    if block > 0 and K % block:
+        K = (K + block - 1) // block * block
+    g = torch.Generator(device=dev).manual_seed(M + N + block)
+    ints = lambda lo, hi, sh: torch.randint(lo, hi, sh, generator=g, device=dev, dtype=torch.int32)  # noqa: E731
+    shape, axis = ((K // block, N), 0) if block > 0 else (((N,), 1) if block == 0 else ((), 1))
+    full = lambda t: t.repeat_interleave(block, 0) if block > 0 else t  # noqa: E731
+    pack = lambda t: torch.nn.functional.pad(t.reshape(-1) & 15, (0, t.numel() % 2)).view(-1, 2)  # noqa: E731
+    nibbles = lambda t: (pack(t)[:, 0] | pack(t)[:, 1] << 4).to(torch.uint8)  # noqa: E731
+    a = ints(-2, 3, (M, K))
+    onehot = torch.zeros((M, K), dtype=torch.float16, device=dev)
+    onehot[torch.arange(M, device=dev), ints(0, K, (M,)).long()] = 1
+    for code, lo in ((olamd.INT4, -8), (olamd.UINT4, 0)):
+        w, z = ints(lo, lo + 16, (K, N)), ints(lo, lo + 16, shape)
+        s2 = torch.pow(2.0, -ints(0, 4, shape).float()).half()
+        rnd = (torch.rand(shape, generator=g, device=dev) * 0.02 + 0.001).half()
+        onnx = nibbles(w)
+        pw = olamd.prepare_weight(onnx, code, (K, N))
+        odd = torch.empty(M * K + 1, dtype=torch.float16, device=dev)[1:].view(M, K)  # 2-byte aligned
+        odd.copy_(a)
+        for zp in (None, z):
+            zb = None if zp is None else nibbles(zp)
+            deq = (w - (0 if zp is None else full(zp))).double() * full(s2).double()
+            want = (a.double() @ deq).to(torch.float32).half()
+            for x in (a.half(), odd):
+                y = olamd.dequantize_linear_matmul(x, pw, s2, zb, axis=axis, x_dtype=code)
+                assert torch.equal(y, want)
+            y = olamd.dequantize_linear_matmul(onehot, pw, rnd, zb, axis=axis, x_dtype=code)
+            general = olamd.dequantize_linear_matmul(onehot, onnx, rnd, zb, axis=axis, x_dtype=code, x_shape=(K, N))
+            assert torch.equal(y, general)
