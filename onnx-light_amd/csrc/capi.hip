@@ -417,12 +417,12 @@ int MatMulInteger(const onnxl_amd_tensor *a, const onnxl_amd_tensor *b,
   // (a_per_row = a_size > 1, :118-119).
   const bool a_vec = a_present && a_count > 1;
   const bool b_vec = b_present && b_count > 1;
-  // Single zero points: read on the host, or under graph capture (no
-  // synchronisation possible) left on the device for the kernels to read.
+  // Single zero points on the device are left there for the kernels to read:
+  // copying them to the host costs a synchronisation per call, and no check
+  // depends on their values.
   const onnxl_amd_tensor *za_t = (a_present && !a_vec && a_count == 1) ? a_zp : nullptr;
   const onnxl_amd_tensor *zb_t = (b_present && !b_vec && b_count == 1) ? b_zp : nullptr;
-  const bool in_place = Capturing(stream);
-  const bool dev_za = in_place && OnDevice(za_t), dev_zb = in_place && OnDevice(zb_t);
+  const bool dev_za = OnDevice(za_t), dev_zb = OnDevice(zb_t);
   int32_t za = 0, zb = 0;
   ReadTwoZeroPoints(stream, dev_za ? nullptr : za_t, dev_zb ? nullptr : zb_t, za, zb);
   p.alpha_scalar = ca - za;
