@@ -213,6 +213,25 @@ void LaunchInt4Gemm(const DqMatMulParams &p, hipStream_t stream) {
   }
 }
 
+// A 4-bit weight in the ONNX packing past its GEMV's rows: tiled into scratch,
+// then as a prepared one.  Never more scratch than the dequantised weight of
+// the general path.  K = 4096, N = 11008: the pass takes 10 us (dequantising it 128),
+// 17 rows 125 -> 22.6 us, 1000 rows 204 -> 119.
+DqMatMulParams WithTiledWeight(const DqMatMulParams &p, const void *scratch) {
+  DqMatMulParams t = p;
+  t.W = static_cast<const uint8_t *>(scratch);
+  t.w_tiled = 1;
+  return t;
+}
+
+bool TilesFirst(const DqMatMulParams &p) {
+  if (p.w_tiled || (p.w_dtype != kInt4 && p.w_dtype != kUint4) || p.K == 0 || p.N % 2 != 0 ||
+      TiledInt4Bytes(p.K, p.N) > p.K * p.N * 2)
+    return false;
+  const DqMatMulParams t = WithTiledWeight(p, reinterpret_cast<const void *>(uintptr_t(256)));
+  return GemvQ4TiledEligible(t) || Int4GemmEligible(t);
+}
+
 }  // namespace
 
 void LaunchHMatMul(const HMatMulParams &p, hipStream_t stream) {
@@ -245,6 +264,7 @@ void LaunchHMatMulBT(const HMatMulParams &p, hipStream_t stream) {
 size_t DqMatMulScratchBytes(const DqMatMulParams &p) {
   if (GemvQ4TiledEligible(p) || Int4GemmEligible(p) || Fp8Eligible(p)) return 0;
   if (GemvQ4Eligible(p)) return GemvQ4ScratchBytes(p);
+  if (TilesFirst(p)) return (size_t)TiledInt4Bytes(p.K, p.N);
   return (size_t)(p.K * p.N) * sizeof(uint16_t);
 }
 
@@ -284,6 +304,14 @@ bool LaunchDqMatMul(const DqMatMulParams &p, void *scratch, size_t scratch_bytes
     if (core && sk::PrefersSkinny(g, false, false)) LaunchF8Skinny(g, stream);
     else if (core && !small) LaunchFp8Gemm(g, stream);
     else LaunchF8Tile(g, /*chain=*/!core, !small, stream);
+    return true;
+  }
+  if (TilesFirst(p)) {
+    if (scratch_bytes < (size_t)TiledInt4Bytes(p.K, p.N)) return false;
+    const DqMatMulParams t = WithTiledWeight(p, scratch);
+    LaunchTileInt4(p.W, p.K, p.N, p.w_dtype == kInt4, static_cast<uint32_t *>(scratch), stream);
+    if (GemvQ4TiledEligible(t)) LaunchGemvQ4Tiled(t, stream);
+    else LaunchInt4Gemm(t, stream);
     return true;
   }
   // general path: dequantise into scratch, then the 16-bit MatMul (K == 0

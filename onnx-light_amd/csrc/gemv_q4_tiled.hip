@@ -336,6 +336,74 @@ __global__ __launch_bounds__(256) void TileInt4Kernel(const uint8_t *x, int64_t 
   out[idx] = word;
 }
 
+// The same for even N: 8 columns x 32 rows per thread.  Bound by the bytes, read
+// and written once: a lane reads 4 bytes of each of its 32 rows (32 lanes a
+// 128-byte line), transposes 8 x 8 nibbles in registers (three rounds of swaps:
+// bytes of different words by v_perm_b32, nibbles by v_bfi_b32) and writes 16
+// bytes per column.  The dword-per-thread kernel gathers every nibble with its
+// own byte load.
+__global__ __launch_bounds__(256) void TileInt4BlockKernel(const uint8_t *x, int64_t K, int64_t N, uint32_t flip,
+                                                           int64_t nh, int64_t ngroups, unsigned gx,
+                                                           v4i *out) {
+  const int64_t h = (int64_t)(blockIdx.x % gx) * 32 + (threadIdx.x & 31);  // columns 8h ... 8h + 7
+  const int64_t gq = (int64_t)(blockIdx.x / gx) * 8 + (threadIdx.x >> 5);
+  const int64_t q = gq >> 2;
+  const int g = (int)(gq & 3);
+  if (h >= nh || q >= ngroups) return;
+  const int64_t n0 = 8 * h, row0 = kGroupRows * q + 8 * g;
+  const uint8_t *src = x + (row0 * N + n0) / 2;
+  const int64_t pitch = N / 2;
+  uint32_t w[4][8];
+  // slot 4 * (j & 1) + j / 2 of w[c]: row row0 + 32 c + j
+  if (n0 + 8 <= N && row0 + 96 + 8 <= K) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) __builtin_memcpy(&w[c][4 * (j & 1) + j / 2], src + (32 * c + j) * pitch, 4);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w[c][j] ^= flip;
+  } else {  // the last rows, the last 2, 4 or 6 columns; past them the offset-binary zero
+    const int bytes = (int)min(int64_t(4), (N - n0) / 2);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        uint32_t d = flip;
+        for (int e = 0; row0 + 32 * c + j < K && e < bytes; ++e)
+          d ^= (uint32_t)src[(32 * c + j) * pitch + e] << (8 * e);
+        w[c][4 * (j & 1) + j / 2] = d;
+      }
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    uint32_t *r = w[c];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {  // halves of words 4 apart
+      const uint32_t a = r[s], b = r[s + 4];
+      r[s] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+      r[s + 4] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {  // bytes of words 2 apart
+      if (s & 2) continue;
+      const uint32_t a = r[s], b = r[s + 2];
+      r[s] = __builtin_amdgcn_perm(b, a, 0x06020400u);
+      r[s + 2] = __builtin_amdgcn_perm(b, a, 0x07030501u);
+    }
+#pragma unroll
+    for (int s = 0; s < 8; s += 2) {  // nibbles of neighbours
+      const uint32_t a = r[s], b = r[s + 1];
+      r[s] = (a & 0x0f0f0f0fu) | ((b << 4) & 0xf0f0f0f0u);
+      r[s + 1] = ((a >> 4) & 0x0f0f0f0fu) | (b & 0xf0f0f0f0u);
+    }
+  }
+  v4i *dst = out + (((h >> 1) * ngroups + q) * 64 + 16 * g + 8 * (h & 1));
+#pragma unroll
+  for (int i = 0; i < 8; ++i) dst[i] = v4i{(int)w[0][i], (int)w[1][i], (int)w[2][i], (int)w[3][i]};
+}
+
 int TilesPerGroup(int64_t ntiles) {
   return (int)std::min<int64_t>(kMaxTiles, std::max<int64_t>(1, (ntiles + kTargetGroups - 1) / kTargetGroups));
 }
@@ -369,6 +437,13 @@ void LaunchTileInt4(const uint8_t *x, int64_t K, int64_t N, int is_signed, uint3
   const int64_t ngroups = (K + kGroupRows - 1) / kGroupRows;
   const int64_t total = TiledInt4Bytes(K, N) / 4;
   if (total == 0) return;
+  const int64_t nh = (N + 15) / 16 * 2, gx = (nh + 31) / 32, blocks = gx * ((ngroups + 1) / 2);
+  if (N % 2 == 0 && blocks <= 0x7fffffff && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+    hipLaunchKernelGGL(TileInt4BlockKernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, K, N,
+                       is_signed ? 0x88888888u : 0u, nh, ngroups, (unsigned)gx,
+                       reinterpret_cast<v4i *>(out));
+    return;
+  }
   hipLaunchKernelGGL(TileInt4Kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, x, K, N,
                      is_signed, ngroups, total, out);
 }

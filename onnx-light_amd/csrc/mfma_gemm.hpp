@@ -1079,6 +1079,15 @@ __global__ __launch_bounds__(kThreads, MB == 2 && (KIND == kBf16F8 || KIND == kF
       const int rr = id / kChunksPerRow, cc = id % kChunksPerRow;
       const bool ok = brow + rr < rcount && cc * (16 / kOsz) < ncol;
       const unsigned at = GRP ? grow[c] + (unsigned)(cc * 16) : ybase + (unsigned)(rr * LDY * kOsz + cc * 16);
+      if constexpr (I4) {
+        if (N % 8 != 0) {  // (N even) the last piece of a row ends inside; rows are 4-byte aligned
+#pragma unroll
+          for (int d = 0; d < 4; ++d)
+            __builtin_amdgcn_raw_buffer_store_b32(piece[c][d], rsY, ok && cc * 8 + 2 * d < ncol ? at + 4 * d : kOob, 0,
+                                                  kStoreThrough);
+          continue;
+        }
+      }
       __builtin_amdgcn_raw_buffer_store_b128(piece[c], rsY, ok ? at : kOob, 0, kStoreThrough);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1134,11 +1143,15 @@ template <int KIND> inline bool PrefersHalfTile(const GemmArgs &p) {
 }
 
 // Eligibility of the 4-bit kernel: as Eligible, with the tiled weight and its
-// scale rows below 2^31 - 2^24 bytes and 4-byte aligned.
+// scale rows below 2^31 - 2^24 bytes and 4-byte aligned, which takes an even N
+// (zero points: a multiple of 8).  An N that is no multiple of 8 stores dwords:
+// 1000 x 4096 x 4098 63 us, 133 through the general path.
 inline bool EligibleI4(const GemmArgs &p) {
   const int64_t lim = (int64_t(1) << 31) - (int64_t(1) << 24);
   auto al = [](const void *q, int n) { return reinterpret_cast<uintptr_t>(q) % n == 0; };
-  return p.K > 0 && p.K % 32 == 0 && p.N % 16 == 0 && p.batch == 1 && al(p.A, 16) && al(p.B, 16) && al(p.Y, 16) &&
+  const bool whole = p.N % 8 == 0;
+  return p.K > 0 && p.K % 32 == 0 && p.N % (p.zp4 ? 8 : 2) == 0 && p.batch == 1 && al(p.A, 16) && al(p.B, 16) &&
+         al(p.Y, whole ? 16 : 4) &&
          al(p.scale, 4) && al(p.zp4, 4) && p.M * p.K * 2 + 4 * kStepBytes < lim && p.M * p.N * 4 < lim &&
          (p.N + 15) / 16 * ((p.K + 127) / 128 + 2) * 1024 < lim && (p.scale_rows + 8) * p.N * 2 < lim;
 }

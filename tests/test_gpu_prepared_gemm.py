@@ -1,10 +1,10 @@
 """Prepared 4-bit weights past 16 rows: the GEMV's 32-row slabs and the GEMM that
 decodes its operand (128- and 256-row tiles), at partial slabs, tiles and K
 steps, every block size, both types, with and without zero points, and operands
-that only the general path takes.  Small integers and power-of-two scales, whose
+that only the general path takes; the ONNX packing, which is tiled first.  Small integers and power-of-two scales, whose
 sums are exact in any order, against 64-bit products; one-hot rows with random
 scales, which give the dequantised weights themselves, bit for bit against the
-general path on the ONNX packing."""
+general path (operands 2 bytes off)."""
 import numpy as np
 import pytest
 import torch
@@ -20,7 +20,7 @@ def dev(olamd):
 
 # rows 17 to 96 are slabs at these sizes, the rest the GEMM
 @pytest.mark.parametrize("M,K,N", [(17, 128, 16), (33, 96, 77), (64, 384, 4112), (97, 256, 8208), (257, 32, 8208),
-                                   (129, 416, 11024), (1500, 224, 2064), (2049, 160, 2176)], ids=str)
+                                   (129, 416, 11024), (1500, 224, 2064), (2049, 160, 2176), (300, 96, 4106), (1300, 64, 2040)], ids=str)
 @pytest.mark.parametrize("block", [8, 32, 64, 128, 0, -1])  # 0: a scale per column, -1: one scale
 def test_prepared_rows(olamd, dev, M, K, N, block):
     if block > 0 and K % block:
@@ -49,6 +49,10 @@ def test_prepared_rows(olamd, dev, M, K, N, block):
             for x in (a.half(), odd):
                 y = olamd.dequantize_linear_matmul(x, pw, s2, zb, axis=axis, x_dtype=code)
                 assert torch.equal(y, want)
+            y = olamd.dequantize_linear_matmul(a.half(), onnx, s2, zb, axis=axis, x_dtype=code, x_shape=(K, N))
+            assert torch.equal(y, want)
             y = olamd.dequantize_linear_matmul(onehot, pw, rnd, zb, axis=axis, x_dtype=code)
-            general = olamd.dequantize_linear_matmul(onehot, onnx, rnd, zb, axis=axis, x_dtype=code, x_shape=(K, N))
+            odd.copy_(onehot)
+            general = olamd.dequantize_linear_matmul(odd, pw, rnd, zb, axis=axis, x_dtype=code)
             assert torch.equal(y, general)
+            odd.copy_(a)
