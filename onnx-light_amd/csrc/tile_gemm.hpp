@@ -97,8 +97,10 @@ __device__ __forceinline__ v4i TailBytes(const char *base, int64_t total, const 
 // registers stay in flight across it (a __syncthreads() would wait for them).
 __device__ __forceinline__ void LdsBarrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-template <int KIND, int SRC, int OUT, bool ZP, int MB, int WB, int D>
-__global__ __launch_bounds__(256, 2) void TileGemmKernel(const GemmArgs p) {
+// G groups of 4 waves: each multiplies its share of the K steps
+// (PrefersTwoGroups).
+template <int KIND, int SRC, int OUT, bool ZP, int MB, int WB, int D, int G>
+__global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void TileGemmKernel(const GemmArgs p) {
   constexpr bool I8 = KIND == mg::kI8;
   constexpr bool BT = SRC == kSrcT, F8 = SRC == kSrcF8 || SRC == kSrcF8Chain;
   static_assert(I8 ? SRC == kSrcRow : !ZP, "int8 B is row-major; zero points are int8's");
@@ -117,10 +119,12 @@ __global__ __launch_bounds__(256, 2) void TileGemmKernel(const GemmArgs p) {
   constexpr int kPitch = kWN * kOsz + 16;           // staged output row
   static_assert(4 * 32 * kPitch <= 2 * kStage, "output staging fits the two stages");
   using Acc = std::conditional_t<I8, v16i, v16f>;
-  __shared__ __align__(16) char sm[2 * kStage];
+  __shared__ __align__(16) char sm[G * 2 * kStage];
   __shared__ int32_t zsum[ZP ? 4 * 2 * kWN : 1];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  char *const sg = sm + grp * 2 * kStage;  // this group's stages
   const int wm = wave >> 1, wn = wave & 1, lr = lane & 31, lg = lane >> 5;
   const int64_t M = p.M, N = p.N, K = p.K;
 
@@ -151,6 +155,9 @@ __global__ __launch_bounds__(256, 2) void TileGemmKernel(const GemmArgs p) {
     nsafe = nk - 1;
     if (!BT && nsafe > 0 && (K - (int64_t)nsafe * kKStep + 1) * NB8 < 16) --nsafe;
   }
+  // this group's plain steps, and the most that one of them has
+  const int s0 = (int)((int64_t)grp * nsafe / G), steps = (int)((int64_t)(grp + 1) * nsafe / G) - s0;
+  const int rounds = (nsafe + G - 1) / G;
   const unsigned aflip = I8 && p.a_u8 ? mg::kFlip : 0u, bflip = I8 && p.b_u8 ? mg::kFlip : 0u;
 
   // ---- addresses of this thread's pieces (K step 0) ----
@@ -194,11 +201,11 @@ __global__ __launch_bounds__(256, 2) void TileGemmKernel(const GemmArgs p) {
   }
 
   v4i fa[D][NA], fb[D][NB];
-  // Step min(t, the last plain step) into register set d: always issued, so
+  // Step min(s0 + t, the last plain step) into register set d: always issued, so
   // that the compiler's waits count exact numbers of younger loads (with a
   // branch around the loads past the end every wait drained them all).
   auto load = [&](int t, int d) __attribute__((always_inline)) {
-    const int64_t tc = t < nsafe ? t : nsafe - 1;
+    const int64_t tc = s0 + t < nsafe ? s0 + t : nsafe - 1;
 #pragma unroll
     for (int q = 0; q < NA; ++q) fa[d][q] = LoadPiece(pa[q] + tc * stepA);
 #pragma unroll
@@ -319,6 +326,11 @@ __global__ __launch_bounds__(256, 2) void TileGemmKernel(const GemmArgs p) {
   auto tail = [&]() __attribute__((always_inline)) {
 #pragma unroll 1
     for (int t = nsafe; t < nk; ++t) {
+      if (G > 1 && grp != 0) {  // the first group's
+        LdsBarrier();
+        LdsBarrier();
+        continue;
+      }
       v4i a[NA], b[NB];
       const int64_t ka = KA - (int64_t)t * 128 - 16 * pc;  // bytes of the row left at this thread's piece
       int64_t nb[NB];                                      // valid bytes of each B piece
@@ -356,22 +368,41 @@ __global__ __launch_bounds__(256, 2) void TileGemmKernel(const GemmArgs p) {
 #pragma unroll
     for (int d = 0; d < D; ++d) load(d, d);
     tail();
-    store(fa[0], fb[0], sm);
+    store(fa[0], fb[0], sg);
     load(D, 0);
     LdsBarrier();
-    for (int t = 0; t < nsafe; t += D) {
+    for (int t = 0; t < rounds; t += D) {
 #pragma unroll
       for (int d = 0; d < D; ++d) {
-        if (t + d >= nsafe) break;
+        if (t + d >= rounds) break;
         const int n = (d + 1) % D;
-        store(fa[n], fb[n], sm + ((d + 1) & 1) * kStage);
+        store(fa[n], fb[n], sg + ((d + 1) & 1) * kStage);
         load(t + d + 1 + D, n);
-        compute(sm + (d & 1) * kStage);
+        if (G == 1 || t + d < steps) compute(sg + (d & 1) * kStage);
         LdsBarrier();
       }
     }
   } else {
     tail();
+  }
+
+  // ---- the groups' sums, added in order by the first through the stages ----
+  if constexpr (G > 1) {
+    static_assert(MB == 1 && WB == 1 && !I8, "one block of fp32 sums per wave");
+    v4f *part = reinterpret_cast<v4f *>(sg) + wave * 4 * 64 + lane;
+    if (grp != 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        part[64 * e] = v4f{acc[0][0][4 * e], acc[0][0][4 * e + 1], acc[0][0][4 * e + 2], acc[0][0][4 * e + 3]};
+    }
+    __syncthreads();
+    if (grp != 0) return;
+#pragma unroll
+    for (int g = 1; g < G; ++g) {
+      const v4f *o = part + g * (2 * kStage / 16);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[0][0][e] += o[64 * (e / 4)][e % 4];
+    }
   }
 
   // ---- zero-point terms (mod 2^32): Y = sum a'b' + beta_j RA_i + alpha_i Q_j, Q_j = CB_j + K beta_j ----
@@ -524,11 +555,37 @@ inline int64_t Tiles(const GemmArgs &p, int side) {
 // fp16; at 688 small tiles the two tie).
 inline bool PrefersSmallTile(const GemmArgs &p, bool core) { return Tiles(p, 64) <= (core ? 256 : 512); }
 
+// Whether the 64 x 64 tile takes two groups of waves per workgroup, each half of
+// the K steps: with at most one tile per CU, one group's step is a chain of LDS
+// writes, a barrier, LDS reads and four dependent MFMAs; two groups fill its
+// waits until the LDS itself is the bound (32 KB read and 16 KB written per
+// step).  The exchange at the end costs about 1 us, so it pays for long K: fp16,
+// one -> two groups, 150 x 4096 outputs at K = 1536 9.5 -> 9.6 us, 2048 11.2 ->
+// 11.2, 3072 16.1 -> 15.3, 4096 22.6 -> 19.4, 8192 40.8 -> 32.9; fp8, whose
+// decode lengthens the chain, 1536 10.4 -> 9.9, 4096 21.4 -> 18.5 us.  int8
+// steps are twice as deep: 4096 12.8 -> 13.4 us.  Four groups were within 0.6 us
+// of two from K = 2048 to 4096 and lost up to 1.4 us below.  With rows of both
+// operands off 16 bytes the loads bound it (fp16 150 x 4097 at K = 4089 29.8 ->
+// 32.7 us).
+template <int KIND, int SRC> inline bool PrefersTwoGroups(const GemmArgs &p) {
+  if (KIND == mg::kI8 || Tiles(p, 64) > 256) return false;
+  if (SRC == kSrcF8 || SRC == kSrcF8Chain) return p.K >= 1536;
+  return p.K >= 3072 && (p.K % 8 == 0 || (SRC == kSrcRow && p.N % 8 == 0));
+}
+
 template <int KIND, int SRC, int OUT, bool ZP> inline void Launch(const GemmArgs &p, bool big, hipStream_t s) {
-  if (big)
-    hipLaunchKernelGGL((TileGemmKernel<KIND, SRC, OUT, ZP, 2, 2, 2>), dim3((unsigned)Tiles(p, 128)), dim3(256), 0, s, p);
-  else
-    hipLaunchKernelGGL((TileGemmKernel<KIND, SRC, OUT, ZP, 1, 1, 4>), dim3((unsigned)Tiles(p, 64)), dim3(256), 0, s, p);
+  if (big) {
+    hipLaunchKernelGGL((TileGemmKernel<KIND, SRC, OUT, ZP, 2, 2, 2, 1>), dim3((unsigned)Tiles(p, 128)), dim3(256), 0, s, p);
+    return;
+  }
+  const dim3 grid((unsigned)Tiles(p, 64));
+  if constexpr (KIND != mg::kI8) {
+    if (PrefersTwoGroups<KIND, SRC>(p)) {
+      hipLaunchKernelGGL((TileGemmKernel<KIND, SRC, OUT, ZP, 1, 1, 4, 2>), grid, dim3(512), 0, s, p);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((TileGemmKernel<KIND, SRC, OUT, ZP, 1, 1, 4, 1>), grid, dim3(256), 0, s, p);
 }
 
 }  // namespace tg

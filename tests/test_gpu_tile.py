@@ -121,3 +121,20 @@ def test_half_tiles(olamd, dev, M, K, N):
     y = olamd.dequantize_linear_grouped_matmul(a.to(torch.bfloat16), e.to(torch.float8_e4m3fn),
                                                torch.ones((2, 1, N), device=dev), idx, cast_to=olamd.BFLOAT16)
     assert torch.equal(y, want.to(torch.float32).to(torch.bfloat16))
+
+
+# Two wave groups per tile (long K, few outputs): K steps that do not split
+# evenly, partial last steps, rows off 16 bytes.
+@pytest.mark.parametrize("M,K,N", [(40, 3072, 64), (64, 3136, 130), (65, 4089, 96), (130, 1536, 72), (33, 3112, 257),
+                                   (7, 1601, 100)], ids=str)
+def test_two_groups(olamd, dev, M, K, N):
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    ints = lambda lo, hi, sh: torch.randint(lo, hi, sh, generator=g, device=dev, dtype=torch.int32)  # noqa: E731
+    a, b = ints(-2, 3, (M, K)), ints(-8, 9, (K, N))
+    exact = a.double() @ b.double()
+    for dt in (torch.float16, torch.bfloat16):
+        assert torch.equal(olamd.matmul(a.to(dt), b.to(dt)), exact.to(torch.float32).to(dt)), dt
+    scale = torch.pow(2.0, -ints(0, 4, (N,)).float())
+    y = olamd.dequantize_linear_matmul(a.to(torch.bfloat16), b.float().to(torch.float8_e4m3fn), scale, None, 1,
+                                       olamd.BFLOAT16)
+    assert torch.equal(y, (exact * scale.double()).to(torch.float32).to(torch.bfloat16))
