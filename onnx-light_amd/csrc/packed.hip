@@ -51,14 +51,18 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t ShareRsrc(void *y, int64_t at,
   return __builtin_amdgcn_make_buffer_rsrc(static_cast<char *>(y) + at, (short)0, bytes, 0x00020000);
 }
 
-template <int OUT> __device__ __forceinline__ void StoreEight(void *y, int64_t i0, const float *v, bool vec) {
+// `share`: the workgroup-sized run of kPkThreads octets that this one, at value
+// i0, belongs to as its thread's.  `numbers`: no value is a NaN.
+template <int OUT>
+__device__ __forceinline__ void StoreEight(void *y, int64_t i0, const float *v, bool vec, int64_t share = blockIdx.x,
+                                           bool numbers = false) {
   constexpr int kBytes = OUT == kFloat ? 32 : 16;  // per thread on the vector paths
   if constexpr (OUT == kFloat) {
     float *dst = static_cast<float *>(y) + i0;
     if (vec) {
       typedef int v4i __attribute__((ext_vector_type(4)));
       const __amdgpu_buffer_rsrc_t rs =
-          ShareRsrc(y, ((int64_t)blockIdx.x * kPkThreads) * kBytes, kPkThreads * kBytes);
+          ShareRsrc(y, share * kPkThreads * kBytes, kPkThreads * kBytes);
       const unsigned off = threadIdx.x * kBytes;
       __builtin_amdgcn_raw_buffer_store_b128(
           v4i{__builtin_bit_cast(int, v[0]), __builtin_bit_cast(int, v[1]), __builtin_bit_cast(int, v[2]),
@@ -76,17 +80,20 @@ template <int OUT> __device__ __forceinline__ void StoreEight(void *y, int64_t i
     for (int e = 0; e < 8; ++e) dst[e] = (double)v[e];
   } else {
     uint16_t h[8];
+    if (OUT == kFloat16 && numbers) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) h[e] = OUT == kFloat16 ? F32ToF16(v[e]) : F32ToBf16(v[e]);
+      for (int e = 0; e < 8; ++e) h[e] = __builtin_bit_cast(uint16_t, (_Float16)v[e]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) h[e] = OUT == kFloat16 ? F32ToF16(v[e]) : F32ToBf16(v[e]);
+    }
     uint16_t *dst = static_cast<uint16_t *>(y) + i0;
     if (vec) {
       typedef int v4i __attribute__((ext_vector_type(4)));
       v4i w;
 #pragma unroll
       for (int k = 0; k < 4; ++k) w[k] = (int)((uint32_t)h[2 * k] | (uint32_t)h[2 * k + 1] << 16);
-      __builtin_amdgcn_raw_buffer_store_b128(w, ShareRsrc(y, ((int64_t)blockIdx.x * kPkThreads) * kBytes,
-                                                          kPkThreads * kBytes),
-                                             threadIdx.x * kBytes, 0, kWriteThrough);
+      __builtin_amdgcn_raw_buffer_store_b128(w, ShareRsrc(y, share * kPkThreads * kBytes, kPkThreads * kBytes), threadIdx.x * kBytes, 0, kWriteThrough);
     } else {
       for (int e = 0; e < 8; ++e) dst[e] = h[e];
     }
@@ -151,30 +158,92 @@ __global__ __launch_bounds__(kPkThreads) void DequantPackedKernel(const uint8_t 
 // The NaN a step produces follows the reference's x86-64 build (SseMul,
 // SseSub of device_codecs.hpp).
 
-__device__ __forceinline__ void DecodeQ4K8(const uint8_t *p, int i0, float v[8]) {
-  const float d = Half2(p), dmin = Half2(p + 2);
-  const uint8_t *sc = p + 4;
-  const int g = i0 >> 5;
-  const int scale = g < 4 ? sc[g] & 63 : (sc[g + 4] & 15) | ((sc[g - 4] >> 6) << 4);
-  const int minimum = g < 4 ? sc[g + 4] & 63 : (sc[g + 4] >> 4) | ((sc[g] >> 6) << 4);
-  const float ds = SseMul(d, (float)scale);
-  const float dm = SseMul(dmin, (float)minimum);
-  const uint8_t *q = p + 16 + (i0 >> 6) * 32 + (i0 & 31);
-  const int sh = 4 * (g & 1);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = SseSub(SseMul(ds, (float)((q[e] >> sh) & 15)), dm);
+// Byte B of a dword as a float in one v_cvt_f32_ubyteB.  Written as
+// (float)((t >> 8B) & 0xff) the compiler folds the byte masks into the
+// mask that isolated the codes and emits a bit-field extract plus
+// v_cvt_f32_ubyte0: two instructions per value instead of one.
+template <int B> __device__ __forceinline__ float UbyteF32(uint32_t t) {
+  float r;
+  if constexpr (B == 0) asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(r) : "v"(t));
+  else if constexpr (B == 1) asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(r) : "v"(t));
+  else if constexpr (B == 2) asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(r) : "v"(t));
+  else asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(r) : "v"(t));
+  return r;
 }
 
-__device__ __forceinline__ void DecodeQ6K8(const uint8_t *p, int i0, float v[8]) {
-  const float d = Half2(p + 208);
-  const float ds = SseMul(d, (float)(int8_t)p[192 + (i0 >> 4)]);
-  const uint8_t *ql = p + (i0 >> 7) * 64 + (i0 & 63);
-  const uint8_t *qh = p + 128 + (i0 >> 7) * 32 + (i0 & 31);
-  const int shl = 4 * ((i0 >> 6) & 1), shh = 2 * ((i0 >> 5) & 3);
-#pragma unroll
-  for (int e = 0; e < 8; ++e)
-    v[e] = SseMul(ds, (float)((((ql[e] >> shl) & 15) | (((qh[e] >> shh) & 3) << 4)) - 32));
+// Four codes, one per byte of t, as floats.
+__device__ __forceinline__ void ByteFloats(uint32_t t, float *f) {
+  f[0] = UbyteF32<0>(t);
+  f[1] = UbyteF32<1>(t);
+  f[2] = UbyteF32<2>(t);
+  f[3] = UbyteF32<3>(t);
 }
+
+__device__ __forceinline__ void NibbleFloats(uint32_t dw, int sh, float *f) { ByteFloats((dw >> sh) & 0x0f0f0f0fu, f); }
+
+__device__ __forceinline__ bool Finite(float x) { return __builtin_fabsf(x) < __builtin_huge_valf(); }
+
+// The bytes of 8 values, and the values from them.
+struct Q4K8 {
+  uint32_t q[2];
+  uint32_t h[4];
+  __device__ __forceinline__ void load(const uint8_t *p, int i0) {
+    __builtin_memcpy(q, p + 16 + (i0 >> 6) * 32 + (i0 & 31), 8);
+    __builtin_memcpy(h, p, 16);
+  }
+  // whether no value is a NaN
+  __device__ __forceinline__ bool decode(int i0, float v[8]) const {
+    const float d = F16ToF32((uint16_t)(h[0] & 0xffffu)), dmin = F16ToF32((uint16_t)(h[0] >> 16));
+    const int g = i0 >> 5, s8 = 8 * (g & 3);
+    const uint32_t b1 = (h[1] >> s8) & 0xffu, b2 = (h[2] >> s8) & 0xffu, b3 = (h[3] >> s8) & 0xffu;
+    const uint32_t scale = g < 4 ? b1 & 63u : (b3 & 15u) | ((b1 >> 6) << 4);
+    const uint32_t minimum = g < 4 ? b2 & 63u : (b3 >> 4) | ((b2 >> 6) << 4);
+    const float ds = SseMul(d, (float)scale);
+    const float dm = SseMul(dmin, (float)minimum);
+    float f[8];
+    NibbleFloats(q[0], 4 * (g & 1), f);
+    NibbleFloats(q[1], 4 * (g & 1), f + 4);
+    const bool numbers = Finite(ds) && Finite(dm);  // |d * scale * q| < 2^26
+    if (numbers) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = ds * f[e] - dm;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = SseSub(SseMul(ds, f[e]), dm);
+    }
+    return numbers;
+  }
+};
+
+struct Q6K8 {
+  uint32_t l[2], h[2];
+  uint16_t d;
+  int8_t sc;
+  __device__ __forceinline__ void load(const uint8_t *p, int i0) {
+    __builtin_memcpy(l, p + (i0 >> 7) * 64 + (i0 & 63), 8);
+    __builtin_memcpy(h, p + 128 + (i0 >> 7) * 32 + (i0 & 31), 8);
+    sc = (int8_t)p[192 + (i0 >> 4)];
+    __builtin_memcpy(&d, p + 208, 2);
+  }
+  // whether no value is a NaN
+  __device__ __forceinline__ bool decode(int i0, float v[8]) const {
+    const float ds = SseMul(F16ToF32(d), (float)sc);
+    const int shl = 4 * ((i0 >> 6) & 1), shh = 2 * ((i0 >> 5) & 3);
+    float f[8];
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      ByteFloats(((l[k] >> shl) & 0x0f0f0f0fu) | ((h[k] >> shh) & 0x03030303u) << 4, f + 4 * k);
+    const bool numbers = Finite(ds);
+    if (numbers) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = ds * (f[e] - 32.f);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = SseMul(ds, f[e] - 32.f);
+    }
+    return numbers;
+  }
+};
 
 template <int TYPE> struct KLayout;
 template <> struct KLayout<10> { static constexpr int bytes = 84; };   // q2_k
@@ -184,23 +253,32 @@ template <> struct KLayout<13> { static constexpr int bytes = 176; };  // q5_k
 template <> struct KLayout<14> { static constexpr int bytes = 210; };  // q6_k
 template <> struct KLayout<23> { static constexpr int bytes = 136; };  // iq4_xs
 
-template <int TYPE> __device__ __forceinline__ void DecodeK8(const uint8_t *p, int i0, float v[8]) {
-  if constexpr (TYPE == 12) DecodeQ4K8(p, i0, v);
-  else DecodeQ6K8(p, i0, v);
-}
+// 32 threads per block, 8 consecutive values each; a workgroup writes
+// kPkRuns runs of 8 * kPkThreads values.  A thread's loads are all on their way
+// before it decodes: with one octet per thread, read byte by byte, a wave's life
+// was its load latency (16.7 M q6_k values to fp16 20.4 us, now 15.2; floor 9.2 at
+// the copy rate).
+constexpr int kPkRuns = 4;
 
-// 32 threads per block, 8 consecutive values each: thread t writes values
-// 8t .. 8t + 7 of the output, as the 32-value kernel does.
 template <int TYPE, int OUT>
 __global__ __launch_bounds__(kPkThreads) void DequantPackedKKernel(const uint8_t *__restrict__ x, int64_t nblocks,
                                                                    void *__restrict__ y, int vec) {
-  const int64_t t = (int64_t)blockIdx.x * kPkThreads + threadIdx.x;
-  if (t >= nblocks * 32) return;
-  const int64_t b = t >> 5;
-  const int i0 = (int)(t & 31) * 8;
-  float v[8];
-  DecodeK8<TYPE>(x + b * KLayout<TYPE>::bytes, i0, v);
-  StoreEight<OUT>(y, b * 256 + i0, v, vec != 0);
+  std::conditional_t<TYPE == 12, Q4K8, Q6K8> raw[kPkRuns];
+  const int i0 = (int)(threadIdx.x & 31) * 8;
+  auto block = [&](int u) { return ((int64_t)blockIdx.x * kPkRuns + u) * (kPkThreads / 32) + (threadIdx.x >> 5); };
+#pragma unroll
+  for (int u = 0; u < kPkRuns; ++u) {
+    const int64_t b = block(u);
+    raw[u].load(x + (b < nblocks ? b : nblocks - 1) * KLayout<TYPE>::bytes, i0);
+  }
+#pragma unroll
+  for (int u = 0; u < kPkRuns; ++u) {
+    const int64_t b = block(u);
+    if (b >= nblocks) return;
+    float v[8];
+    const bool numbers = raw[u].decode(i0, v);
+    StoreEight<OUT>(y, b * 256 + i0, v, vec != 0, (int64_t)blockIdx.x * kPkRuns + u, numbers);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -437,7 +515,8 @@ template <int TYPE> void LaunchPkXOut(const uint8_t *x, int64_t nblocks, int out
 }
 
 template <int TYPE> void LaunchPkKOut(const uint8_t *x, int64_t nblocks, int out, void *y, int vec, hipStream_t s) {
-  const dim3 g((unsigned)((nblocks * 32 + kPkThreads - 1) / kPkThreads));
+  const int64_t per = kPkRuns * (kPkThreads / 32);  // blocks per workgroup
+  const dim3 g((unsigned)((nblocks + per - 1) / per));
   switch (out) {
   case kFloat: hipLaunchKernelGGL((DequantPackedKKernel<TYPE, kFloat>), g, dim3(kPkThreads), 0, s, x, nblocks, y, vec); break;
   case kFloat16: hipLaunchKernelGGL((DequantPackedKKernel<TYPE, kFloat16>), g, dim3(kPkThreads), 0, s, x, nblocks, y, vec); break;
@@ -533,6 +612,51 @@ __device__ __forceinline__ void StageRows(uint32_t *stage, const uint8_t *src, i
   }
 }
 
+// The sums over a wave's lanes of its 4 outputs from n0 and M rows of A, rounded
+// and stored.  A step that adds across lanes also halves the values a lane still
+// holds (rows, then activation rows, padded to a power of two): 7 exchanges for
+// M = 1 and 32 for M = 8, where adding each value across all lanes by itself
+// takes 24 and 192 (q4_k, 4096 outputs, K = 512: M = 1 3.8 -> 3.2 us, M = 8 10.8 ->
+// 4.3; 14336 outputs, M = 8 22.0 -> 8.9).
+template <int C, int O> __device__ __forceinline__ float FoldLanes(const float (&s)[C], int lane, int &m) {
+  if constexpr (O == 0) {
+    static_assert(C == 1, "at most 8 values over 16 lanes");
+    return s[0];
+  } else if constexpr (C == 1) {
+    const float t[1] = {s[0] + __shfl_xor(s[0], O)};
+    return FoldLanes<1, O / 2>(t, lane, m);
+  } else {
+    float t[C / 2];
+    const bool up = lane & O;
+#pragma unroll
+    for (int i = 0; i < C / 2; ++i) t[i] = (up ? s[C / 2 + i] : s[i]) + __shfl_xor(up ? s[i] : s[C / 2 + i], O);
+    m += up ? C / 2 : 0;
+    return FoldLanes<C / 2, O / 2>(t, lane, m);
+  }
+}
+template <int M>
+__device__ __forceinline__ void StoreRowSums(const float (&acc)[4][M], int lane, int64_t n0, int64_t N,
+                                             uint16_t *__restrict__ y) {
+  constexpr int C = M > 4 ? 8 : (M > 2 ? 4 : M);
+  float s[C];
+#pragma unroll
+  for (int m = 0; m < C; ++m) {
+    if (m >= M) {
+      s[m] = 0.f;
+      continue;
+    }
+    float r[2];
+    const bool up = lane & 32, odd = lane & 16;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) r[i] = (up ? acc[2 + i][m] : acc[i][m]) + __shfl_xor(up ? acc[i][m] : acc[2 + i][m], 32);
+    s[m] = (odd ? r[1] : r[0]) + __shfl_xor(odd ? r[0] : r[1], 16);
+  }
+  int m = 0;
+  const float v = FoldLanes<C, 8>(s, lane, m);
+  const int64_t n = n0 + (lane >> 4);
+  if ((lane & (16 / C - 1)) == 0 && m < M && n < N) y[m * N + n] = F32ToF16(v);
+}
+
 template <int M>
 __global__ __launch_bounds__(256) void GemvQ40Kernel(const uint16_t *__restrict__ a, const uint8_t *__restrict__ w,
                                                      int64_t N, int64_t K, uint16_t *__restrict__ y) {
@@ -616,17 +740,7 @@ __global__ __launch_bounds__(256) void GemvQ40Kernel(const uint16_t *__restrict_
     }
     __syncthreads();  // the stage is rewritten by the next chunk
   }
-#pragma unroll
-  for (int c = 0; c < kGvCols; ++c) {
-    const int64_t n = n0 + wave * kGvCols + c;
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      float s = acc[c][m];
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
-      if (lane == 0 && n < N) y[m * N + n] = F32ToF16(s);
-    }
-  }
+  StoreRowSums(acc, lane, n0 + wave * kGvCols, N, y);
 }
 
 // Fused q8_0 GEMV, as the q4_0 one: y[m, n] = sum_k a[m, k] * W[n, k] with W
@@ -701,17 +815,7 @@ __global__ __launch_bounds__(256) void GemvQ80Kernel(const uint16_t *__restrict_
     }
     __syncthreads();  // the stage is rewritten by the next chunk
   }
-#pragma unroll
-  for (int c = 0; c < kGvCols; ++c) {
-    const int64_t n = n0 + wave * kGvCols + c;
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      float s = acc[c][m];
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
-      if (lane == 0 && n < N) y[m * N + n] = F32ToF16(s);
-    }
-  }
+  StoreRowSums(acc, lane, n0 + wave * kGvCols, N, y);
 }
 
 // Streamed q4_0 / q8_0 GEMV for K % 256 == 0 (every row starts 16-byte
@@ -889,17 +993,7 @@ __global__ __launch_bounds__(64) void GemvQ0StreamKernel(const uint16_t *__restr
   };
   for (int c = 0; c + 1 < nchunks; ++c) chunk(c, std::true_type{});
   chunk(nchunks - 1, std::false_type{});
-#pragma unroll
-  for (int r = 0; r < kQsRows; ++r) {
-    const int64_t n = n0 + r;
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      float s = acc[r][m];
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
-      if (lane == 0 && n < N) y[m * N + n] = F32ToF16(s);
-    }
-  }
+  StoreRowSums(acc, lane, n0, N, y);
 }
 
 // The streamed kernel's conditions: 16-byte aligned operands, K % 256 == 0,
@@ -936,29 +1030,6 @@ void LaunchGemvQ0Stream(const uint16_t *a, const uint8_t *w, int64_t M, int64_t 
 // bytes; every block starts 16-byte aligned as 144 = 9 x 16) and one 8-byte
 // run of codes; q6_k (210-byte blocks, 2-byte aligned) four 16-bit loads of
 // low nibbles, four of high bits, the sub-block's scale byte and d.
-// Byte B of a dword as a float in one v_cvt_f32_ubyteB.  Written as
-// (float)((t >> 8B) & 0xff) the compiler folds the byte masks into the
-// mask that isolated the codes and emits a bit-field extract plus
-// v_cvt_f32_ubyte0: two instructions per value instead of one.
-template <int B> __device__ __forceinline__ float UbyteF32(uint32_t t) {
-  float r;
-  if constexpr (B == 0) asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(r) : "v"(t));
-  else if constexpr (B == 1) asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(r) : "v"(t));
-  else if constexpr (B == 2) asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(r) : "v"(t));
-  else asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(r) : "v"(t));
-  return r;
-}
-
-// Four codes, one per byte of t, as floats.
-__device__ __forceinline__ void ByteFloats(uint32_t t, float *f) {
-  f[0] = UbyteF32<0>(t);
-  f[1] = UbyteF32<1>(t);
-  f[2] = UbyteF32<2>(t);
-  f[3] = UbyteF32<3>(t);
-}
-
-__device__ __forceinline__ void NibbleFloats(uint32_t dw, int sh, float *f) { ByteFloats((dw >> sh) & 0x0f0f0f0fu, f); }
-
 // The raw bytes one lane needs from one block, loaded a block ahead of use.
 template <int TYPE> struct KRaw;
 template <> struct KRaw<12> {
@@ -1272,17 +1343,7 @@ __global__ __launch_bounds__(256) void GemvKKernel(const uint16_t *__restrict__ 
 #pragma unroll
     for (int m = 0; m < M; ++m) av[m] = avn[m];
   }
-#pragma unroll
-  for (int c = 0; c < kGvCols; ++c) {
-    const int64_t n = n0 + c;
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      float s = acc[c][m];
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
-      if (lane == 0 && n < N) y[m * N + n] = F32ToF16(s);
-    }
-  }
+  StoreRowSums(acc, lane, n0, N, y);
 }
 
 // The same GEMV with the weight streamed through LDS.  Per lane, the direct
@@ -1410,17 +1471,130 @@ __global__ __launch_bounds__(256) void GemvKLdsKernel(const uint16_t *__restrict
     if (s + 1 < nstages) put(buf ^ 1);  // the other buffer: every wave left it at the last barrier
     __syncthreads();
   }
+  StoreRowSums(acc, lane, n0 + wave * kGvCols, N, y);
+}
+
+// q4_k, up to kQ4kRows activation rows: 16 code bytes per lane (8 lanes per
+// block), both nibbles of each, so a lane decodes two scales for 32 values.  The
+// staged kernel is bound by its VALU work: 8 values per lane cost a whole scale
+// decode, and each code an extract and a conversion of its own.  Here a masked
+// dword is a pair of codes as fp16 denormals (q * 2^-24; the high nibbles
+// q * 2^-20), which the mixed-precision multiply-add takes as it is, its fp32
+// scale carrying the power of two: exact, so the rounding stays that of DecodeK.
+// Per 8 values 5 extracts, 8 multiply-adds and 4 dot products; those bound it.
+// The header's dwords go to the lanes of a quad, one each, and round by DPP.
+constexpr int kQ4kRows = 4;
+// Where most of a wave's 8 blocks per step are there.  Staged kernel against this
+// one, N = 14336 / 4096, M = 1: K = 4096 16.5 -> 14.3 / 8.4 -> 6.1 us, 2816 13.1 ->
+// 12.7 / 6.9 -> 5.7, 2304 (9 blocks) 11.5 -> 12.6 / 6.2 -> 5.8, 1536 8.4 -> 7.8 /
+// 4.8 -> 3.6, 1024 6.4 -> 7.1; M = 4: 4096 20.1 -> 19.1 / 9.5 -> 8.0, 2048 12.0 ->
+// 12.0 / 6.3 -> 5.1, 2816 15.9 -> 18.1; M = 8: 4096 29.0 -> 36.7.
+inline bool PrefersQ4K(int64_t M, int64_t nb) {
+  return nb % 8 == 0 || (M == 1 && 3 * nb >= 16 * ((nb + 7) / 8));
+}
+// x of lane L of each four lanes
+template <int L> __device__ __forceinline__ uint32_t QuadLane(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x55 * L, 0xf, 0xf, true);
+}
+
+template <int M>
+__global__ __launch_bounds__(256) void GemvQ4KKernel(const uint16_t *__restrict__ a, const uint8_t *__restrict__ w,
+                                                     int64_t N, int64_t K, uint16_t *__restrict__ y) {
+  typedef unsigned v4u __attribute__((ext_vector_type(4)));
+  constexpr int kBytes = KLayout<12>::bytes;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sub = lane >> 3, o = lane & 7, j = o >> 1;
+  const int nb = (int)(K / 256);
+  const int64_t n0 = (int64_t)blockIdx.x * kGvRows + wave * kGvCols;
+  const uint8_t *row[kGvCols];  // rows past N read the last and are not stored
 #pragma unroll
-  for (int c = 0; c < kGvCols; ++c) {
-    const int64_t n = n0 + wave * kGvCols + c;
+  for (int c = 0; c < kGvCols; ++c) row[c] = w + (n0 + c < N ? n0 + c : N - 1) * nb * kBytes;
+  float acc[kGvCols][M];
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-      float s = acc[c][m];
+  for (int c = 0; c < kGvCols; ++c)
 #pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
-      if (lane == 0 && n < N) y[m * N + n] = F32ToF16(s);
+    for (int m = 0; m < M; ++m) acc[c][m] = 0.f;
+  unsigned hd[2][kGvCols];  // dword o % 4 of the block's header
+  v4u q[2][kGvCols];
+  // blocks 8 t + sub (past the row: its last, not computed)
+  auto load = [&](int t, int s) __attribute__((always_inline)) {
+    const unsigned at = (unsigned)min(8 * t + sub, nb - 1) * kBytes;
+#pragma unroll
+    for (int c = 0; c < kGvCols; ++c) {
+      hd[s][c] = __builtin_nontemporal_load(reinterpret_cast<const unsigned *>(row[c] + at) + (o & 3));
+      q[s][c] = __builtin_nontemporal_load(reinterpret_cast<const v4u *>(row[c] + at + 16 + 16 * o));
     }
+  };
+  const int sh = 16 * (j & 1);
+  // sub-blocks 0 to 3 take six bits of one byte, 4 to 7 four and two of others
+  const uint32_t m6 = j < 2 ? 0x3f3fu : 0u, m4 = j < 2 ? 0u : 0x0f0fu, m2 = j < 2 ? 0u : 0x3030u;
+  // step t from set s; with `more`, step t + 1 into the other set behind this
+  // step's activations, whose wait then covers none of its loads
+  auto step = [&](int t, int s, bool more) __attribute__((always_inline)) {
+    v4u av[M][2][2];
+    const uint16_t *at = a + (int64_t)min(8 * t + sub, nb - 1) * 256 + 64 * j + 16 * (o & 1);
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) av[m][h][e] = *reinterpret_cast<const v4u *>(at + m * K + 32 * h + 8 * e);
+    if (more) load(t + 1, s ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    // the activations of the 16 low and the 16 high nibbles, in the codes'
+    // pairs: (0, 2), (1, 3) of every four
+    uint32_t ap[M][2][8];
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const v4u x = av[m][h][e];
+#pragma unroll
+          for (int d = 0; d < 2; ++d) {
+            ap[m][h][4 * e + 2 * d] = __builtin_amdgcn_perm(x[2 * d + 1], x[2 * d], 0x05040100u);
+            ap[m][h][4 * e + 2 * d + 1] = __builtin_amdgcn_perm(x[2 * d + 1], x[2 * d], 0x07060302u);
+          }
+        }
+    if (8 * t + sub < nb) {
+#pragma unroll
+      for (int c = 0; c < kGvCols; ++c) {
+        const uint32_t h0 = QuadLane<0>(hd[s][c]), h1 = QuadLane<1>(hd[s][c]), h2 = QuadLane<2>(hd[s][c]),
+                       h3 = QuadLane<3>(hd[s][c]);
+        const float d = F16ToF32((uint16_t)(h0 & 0xffffu)), dmin = F16ToF32((uint16_t)(h0 >> 16));
+        // scale and minimum bytes of sub-blocks 2 j and 2 j + 1 (DecodeK)
+        const uint32_t b1 = h1 >> sh, b2 = h2 >> sh, b3 = h3 >> sh;
+        const uint32_t sc = (b1 & m6) | (b3 & m4) | ((b1 >> 2) & m2);
+        const uint32_t mn = (b2 & m6) | ((b3 >> 4) & m4) | ((b2 >> 2) & m2);
+        const float ds[2] = {d * UbyteF32<0>(sc) * 0x1p24f, d * UbyteF32<1>(sc) * 0x1p20f};
+        const float dm[2] = {dmin * UbyteF32<0>(mn), dmin * UbyteF32<1>(mn)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t x = q[s][c][e], x8 = x >> 8;
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              const h2_t k = AsH2((u ? x8 : x) & (h ? 0x00f000f0u : 0x000f000fu));
+              const h2_t v = h2_t{(_Float16)__builtin_fmaf((float)k.x, ds[h], -dm[h]),
+                                  (_Float16)__builtin_fmaf((float)k.y, ds[h], -dm[h])};
+#pragma unroll
+              for (int m = 0; m < M; ++m) acc[c][m] = __builtin_amdgcn_fdot2(AsH2(ap[m][h][2 * e + u]), v, acc[c][m], false);
+            }
+        }
+      }
+    }
+  };
+  const int nt = (nb + 7) / 8;
+  load(0, 0);
+  for (int t = 0; t + 1 < nt; t += 2) {
+    step(t, 0, true);
+    if (t + 2 < nt) step(t + 1, 1, true);
+    else step(t + 1, 1, false);
   }
+  if (nt & 1) step(nt - 1, 0, false);
+  StoreRowSums(acc, lane, n0, N, y);
 }
 
 // Blocks per stage: about 10-18 KB of weight per stage for 16 rows, fewer
@@ -1434,6 +1608,12 @@ template <int TYPE, int M> constexpr int KStageBlocks() {
 template <int TYPE, int M>
 void LaunchGemvKM(const uint16_t *a, const uint8_t *w, int64_t N, int64_t K, uint16_t *y, hipStream_t s) {
   const dim3 g((unsigned)((N + kGvRows - 1) / kGvRows));
+  if constexpr (TYPE == 12 && M <= kQ4kRows) {
+    if (PrefersQ4K(M, K / 256)) {
+      hipLaunchKernelGGL(GemvQ4KKernel<M>, g, dim3(256), 0, s, a, w, N, K, y);
+      return;
+    }
+  }
   if (N * (K / 256) * KLayout<TYPE>::bytes < (int64_t(1) << 31) - (int64_t(1) << 20))
     hipLaunchKernelGGL((GemvKLdsKernel<TYPE, M, KStageBlocks<TYPE, M>()>), g, dim3(256), 0, s, a, w, N, K, y);
   else

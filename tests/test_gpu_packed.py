@@ -137,6 +137,14 @@ _GEMV_SHAPES = [(1, 96, 64), (3, 200, 256), (8, 64, 4096), (2, 1000, 1024), (1, 
                 (4, 129, 6144), (1, 37, 256), (2, 129, 6144), (1, 1024, 14336), (2, 6, 8448)]
 
 
+# q4_k with 16 code bytes per lane: whole and partial steps of 8 blocks, outputs
+# that end inside a wave's four and a workgroup's 16.
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1536), (1, 18, 2048), (1, 35, 2816), (2, 5, 2048), (3, 17, 4096),
+                                   (4, 33, 2048), (1, 3, 4352)])
+def test_q4k_gemv_wide(olamd, oracle, dev, M, N, K):
+    test_k_quant_gemv_vs_chain(olamd, oracle, dev, "gguf:q4_k", M, N, K)
+
+
 @pytest.mark.parametrize("fmt,block_bytes", [("gguf:q4_0", 18), ("gguf:q8_0", 34)])
 @pytest.mark.parametrize("M,N,K", _GEMV_SHAPES)
 def test_packed_gemv_vs_chain(olamd, oracle, dev, fmt, block_bytes, M, N, K):
