@@ -1,10 +1,11 @@
 """Prepared 4-bit weights past 16 rows: the GEMV's 32-row slabs and the GEMM that
 decodes its operand (128- and 256-row tiles), at partial slabs, tiles and K
-steps, every block size, both types, with and without zero points, and operands
-that only the general path takes; the ONNX packing, which is tiled first.  Small integers and power-of-two scales, whose
-sums are exact in any order, against 64-bit products; one-hot rows with random
-scales, which give the dequantised weights themselves, bit for bit against the
-general path (operands 2 bytes off)."""
+steps, every block size, both types, with and without zero points, operands that
+only the general path takes, and the ONNX packing, which is tiled first.  Small
+integers and power-of-two scales, whose sums are exact in any order, against
+64-bit products; one-hot rows with random scales, which give the dequantised
+weights themselves, bit for bit against the general path (operands 2 bytes off)
+and, for that path, against fp32 arithmetic rounded once."""
 import numpy as np
 import pytest
 import torch
@@ -56,3 +57,35 @@ def test_prepared_rows(olamd, dev, M, K, N, block):
             general = olamd.dequantize_linear_matmul(odd, pw, rnd, zb, axis=axis, x_dtype=code)
             assert torch.equal(y, general)
             odd.copy_(a)
+
+
+@pytest.mark.parametrize("K,N,block", [(8, 8, 8), (264, 24, 8), (96, 648, 32), (264, 1032, 88), (100, 72, 4),
+                                       (130, 20, 65), (257, 16, 0), (300, 77, -1)], ids=str)
+@pytest.mark.parametrize("bf16", [False, True])
+def test_general_weights(olamd, dev, K, N, block, bf16):
+    """The general path's dequantisation, value by value: the identity as
+    activations (bf16 with FLOAT scales and a Cast, or fp16 2 bytes off), every
+    weight type, row-major and tiled, whole and partial groups of rows and columns."""
+    g = torch.Generator(device=dev).manual_seed(K + N + block)
+    ints = lambda lo, hi, sh: torch.randint(lo, hi, sh, generator=g, device=dev, dtype=torch.int32)  # noqa: E731
+    dt = torch.bfloat16 if bf16 else torch.float16
+    a = torch.empty(K * K + 1, dtype=dt, device=dev)[1:].view(K, K)
+    a.copy_(torch.eye(K, device=dev))
+    shape, axis = ((K // block, N), 0) if block > 0 else (((N,), 1) if block == 0 else ((), 1))
+    full = lambda t: t.repeat_interleave(block, 0) if block > 0 else t  # noqa: E731
+    pack = lambda t: torch.nn.functional.pad(t.reshape(-1) & 15, (0, t.numel() % 2)).view(-1, 2)  # noqa: E731
+    nibbles = lambda t: (pack(t)[:, 0] | pack(t)[:, 1] << 4).to(torch.uint8)  # noqa: E731
+    scale = torch.rand(shape, generator=g, device=dev) * 0.02 + 0.001
+    scale = scale if bf16 else scale.half()
+    kw = dict(axis=axis, cast_to=olamd.BFLOAT16 if bf16 else 0)
+    for code, lo, bits in ((olamd.INT8, -128, 8), (olamd.UINT8, 0, 8), (olamd.INT4, -8, 4), (olamd.UINT4, 0, 4)):
+        w, z = ints(lo, lo + (1 << bits), (K, N)), ints(lo, lo + (1 << bits), shape)
+        for zp in (None, z):
+            want = ((w - (0 if zp is None else full(zp))).float() * full(scale).float()).to(dt)
+            store = nibbles if bits == 4 else (lambda t: t.to(torch.int8 if lo else torch.uint8))  # noqa: E731
+            zb = None if zp is None else store(zp)
+            y = olamd.dequantize_linear_matmul(a, store(w), scale, zb, x_dtype=code, x_shape=(K, N), **kw)
+            assert torch.equal(y, want)
+            if bits == 4:
+                pw = olamd.prepare_weight(nibbles(w), code, (K, N))
+                assert torch.equal(olamd.dequantize_linear_matmul(a, pw, scale, zb, x_dtype=code, **kw), want)
