@@ -4,7 +4,8 @@
 //
 // Workgroup: 4 waves (2 x 2), tile (64 MB) x (64 WB), each wave MB x WB blocks
 // of 32 x 32.  MB = WB = 2 (128 x 128) where those tiles fill the chip, else
-// MB = WB = 1 (64 x 64), which puts four times the workgroups on it.
+// MB = WB = 1 (64 x 64), which puts four times the workgroups on it, or MB = 1,
+// WB = 2 between the two (PrefersWideTile).
 //
 // Memory path.  Both operands go global -> registers -> LDS.  The core's
 // direct loads need 16-byte aligned rows; a register load does not, so a row
@@ -573,10 +574,27 @@ template <int KIND, int SRC> inline bool PrefersTwoGroups(const GemmArgs &p) {
   return p.K >= 3072 && (p.K % 8 == 0 || (SRC == kSrcRow && p.N % 8 == 0));
 }
 
+// Whether 64 x 128 tiles take a problem of more 64 x 64 tiles than CUs: at most
+// one per CU, they keep any CU from two of the small ones, whose LDS traffic (48
+// KB a step, against 72 for twice the outputs) does not overlap.  335 x 3001
+// outputs, 64 x 64 -> 64 x 128: int8 K = 513 11.2 -> 8.8 us, 1001 13.0 -> 10.4, 4090
+// 29.3 -> 25.2; fp16 11.3 -> 10.2, 15.3 -> 13.1, 42.5 -> 35.2.  Steps in flight: two
+// for int8 (four: 9.9, 11.5, 25.0), four for fp16 (two: 9.7, 12.7, 39.2).  fp8 weights
+// stay with the small tile (K = 1001 14.6 -> 14.9, 4090 38.1 -> 40.7).
+inline int64_t WideTiles(const GemmArgs &p) { return (p.M + 63) / 64 * ((p.N + 127) / 128) * p.batch; }
+inline bool PrefersWideTile(const GemmArgs &p) { return Tiles(p, 64) > 256 && WideTiles(p) <= 256; }
+
 template <int KIND, int SRC, int OUT, bool ZP> inline void Launch(const GemmArgs &p, bool big, hipStream_t s) {
   if (big) {
     hipLaunchKernelGGL((TileGemmKernel<KIND, SRC, OUT, ZP, 2, 2, 2, 1>), dim3((unsigned)Tiles(p, 128)), dim3(256), 0, s, p);
     return;
+  }
+  if constexpr (SRC == kSrcRow || SRC == kSrcT) {
+    if (PrefersWideTile(p)) {
+      hipLaunchKernelGGL((TileGemmKernel<KIND, SRC, OUT, ZP, 1, 2, KIND == mg::kI8 ? 2 : 4, 1>),
+                         dim3((unsigned)WideTiles(p)), dim3(256), 0, s, p);
+      return;
+    }
   }
   const dim3 grid((unsigned)Tiles(p, 64));
   if constexpr (KIND != mg::kI8) {

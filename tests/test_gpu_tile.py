@@ -138,3 +138,18 @@ def test_two_groups(olamd, dev, M, K, N):
     y = olamd.dequantize_linear_matmul(a.to(torch.bfloat16), b.float().to(torch.float8_e4m3fn), scale, None, 1,
                                        olamd.BFLOAT16)
     assert torch.equal(y, (exact * scale.double()).to(torch.float32).to(torch.bfloat16))
+
+
+# 64 x 128 tiles: more small tiles than CUs, rows and columns that end inside one.
+@pytest.mark.parametrize("M,K,N", [(65, 130, 8250), (330, 333, 3137), (1040, 65, 1023), (63, 2049, 16500)], ids=str)
+def test_wide_tiles(olamd, dev, M, K, N):
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    ints = lambda lo, hi, sh: torch.randint(lo, hi, sh, generator=g, device=dev, dtype=torch.int32)  # noqa: E731
+    a, b = ints(0, 256, (M, K)).to(torch.uint8), ints(-128, 128, (K, N)).to(torch.int8)
+    za, zb = ints(0, 256, (M,)).to(torch.uint8), ints(-128, 128, (N,)).to(torch.int8)
+    assert torch.equal(olamd.matmul_integer(a, b).double(), a.double() @ b.double())
+    y = olamd.matmul_integer(a, b, za, zb)
+    assert torch.equal(y.double(), (a.double() - za.double().unsqueeze(1)) @ (b.double() - zb.double()))
+    a, b = ints(-2, 3, (M, K)), ints(-8, 9, (K, N))
+    for dt in (torch.float16, torch.bfloat16):
+        assert torch.equal(olamd.matmul(a.to(dt), b.to(dt)), (a.double() @ b.double()).to(torch.float32).to(dt)), dt
