@@ -580,21 +580,29 @@ template <int KIND, int SRC> inline bool PrefersTwoGroups(const GemmArgs &p) {
 // outputs, 64 x 64 -> 64 x 128: int8 K = 513 11.2 -> 8.8 us, 1001 13.0 -> 10.4, 4090
 // 29.3 -> 25.2; fp16 11.3 -> 10.2, 15.3 -> 13.1, 42.5 -> 35.2.  Steps in flight: two
 // for int8 (four: 9.9, 11.5, 25.0), four for fp16 (two: 9.7, 12.7, 39.2).  fp8 weights
-// stay with the small tile (K = 1001 14.6 -> 14.9, 4090 38.1 -> 40.7).
+// stay with the small tile (K = 1001 14.6 -> 14.9, 4090 38.1 -> 40.7).  Two of them
+// per CU also beat two rounds of 128 x 128 ones, which rows or columns left over
+// fill badly: 300 x 11007, 128 x 128 -> 64 x 128, int8 K = 1001 21.9 -> 16.1 us, 4090
+// 59.6 -> 41.8, fp16 31.8 -> 22.7 and 82.5 -> 61.1; against one round they lose (1000 x
+// 3001 at K = 4090 37.9 -> 41.3, 57.2 -> 60.1), three rounds against two too (1500 x
+// 4001 60.7 -> 66.9).
 inline int64_t WideTiles(const GemmArgs &p) { return (p.M + 63) / 64 * ((p.N + 127) / 128) * p.batch; }
-inline bool PrefersWideTile(const GemmArgs &p) { return Tiles(p, 64) > 256 && WideTiles(p) <= 256; }
+inline bool PrefersWideTile(const GemmArgs &p) {
+  const int64_t wide = WideTiles(p);
+  return (Tiles(p, 64) > 256 && wide <= 256) || (Tiles(p, 128) > 256 && wide <= 512);
+}
 
 template <int KIND, int SRC, int OUT, bool ZP> inline void Launch(const GemmArgs &p, bool big, hipStream_t s) {
-  if (big) {
-    hipLaunchKernelGGL((TileGemmKernel<KIND, SRC, OUT, ZP, 2, 2, 2, 1>), dim3((unsigned)Tiles(p, 128)), dim3(256), 0, s, p);
-    return;
-  }
   if constexpr (SRC == kSrcRow || SRC == kSrcT) {
     if (PrefersWideTile(p)) {
       hipLaunchKernelGGL((TileGemmKernel<KIND, SRC, OUT, ZP, 1, 2, KIND == mg::kI8 ? 2 : 4, 1>),
                          dim3((unsigned)WideTiles(p)), dim3(256), 0, s, p);
       return;
     }
+  }
+  if (big) {
+    hipLaunchKernelGGL((TileGemmKernel<KIND, SRC, OUT, ZP, 2, 2, 2, 1>), dim3((unsigned)Tiles(p, 128)), dim3(256), 0, s, p);
+    return;
   }
   const dim3 grid((unsigned)Tiles(p, 64));
   if constexpr (KIND != mg::kI8) {

@@ -140,8 +140,10 @@ def test_two_groups(olamd, dev, M, K, N):
     assert torch.equal(y, (exact * scale.double()).to(torch.float32).to(torch.bfloat16))
 
 
-# 64 x 128 tiles: more small tiles than CUs, rows and columns that end inside one.
-@pytest.mark.parametrize("M,K,N", [(65, 130, 8250), (330, 333, 3137), (1040, 65, 1023), (63, 2049, 16500)], ids=str)
+# 64 x 128 tiles: more small tiles than CUs, or more large ones; rows and columns
+# that end inside one.
+@pytest.mark.parametrize("M,K,N", [(65, 130, 8250), (330, 333, 3137), (1040, 65, 1023), (63, 2049, 16500),
+                                   (300, 129, 11007)], ids=str)
 def test_wide_tiles(olamd, dev, M, K, N):
     g = torch.Generator(device=dev).manual_seed(M + K)
     ints = lambda lo, hi, sh: torch.randint(lo, hi, sh, generator=g, device=dev, dtype=torch.int32)  # noqa: E731
