@@ -22,6 +22,7 @@
 #pragma once
 
 #include "mfma_gemm.hpp"
+#include "tile_steps.hpp"
 
 namespace onnxl_amd {
 namespace tg {
@@ -147,15 +148,9 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void TileGemmKernel(const 
   const int64_t NB8 = BT ? K * kBsz : N * kBsz;   // bytes of a B row as it lies in memory
   const int64_t a_total = M * KA, b_total = (BT ? N : K) * NB8;
   const int nk = (int)((K + kKStep - 1) / kKStep);
-  // Steps read with plain loads: every piece ends inside the matrix (one of a
-  // row-major B may cross into the next rows), and no k lies past K.  The
-  // others, at most two, are multiplied first, while the loads of the first
-  // plain steps are on their way.
-  int nsafe = nk;
-  if (K % kKStep != 0 || (!BT && NB8 % 16 != 0)) {
-    nsafe = nk - 1;
-    if (!BT && nsafe > 0 && (K - (int64_t)nsafe * kKStep + 1) * NB8 < 16) --nsafe;
-  }
+  // Steps read with plain loads.  The others, at most two, are multiplied
+  // first, while the loads of the first plain steps are on their way.
+  const int nsafe = PlainSteps(K, kKStep, !BT, NB8);
   // this group's plain steps, and the most that one of them has
   const int s0 = (int)((int64_t)grp * nsafe / G), steps = (int)((int64_t)(grp + 1) * nsafe / G) - s0;
   const int rounds = (nsafe + G - 1) / G;

@@ -155,3 +155,24 @@ def test_wide_tiles(olamd, dev, M, K, N):
     a, b = ints(-2, 3, (M, K)), ints(-8, 9, (K, N))
     for dt in (torch.float16, torch.bfloat16):
         assert torch.equal(olamd.matmul(a.to(dt), b.to(dt)), (a.double() @ b.double()).to(torch.float32).to(dt)), dt
+
+
+# K = 0: nothing is read, sums are zero (rows of whole 16-byte pieces and others).
+@pytest.mark.parametrize("M,N", [(3, 15), (8, 16), (1, 1), (70, 130), (600, 2053)], ids=str)
+def test_empty_k(olamd, dev, M, N):
+    empty = lambda *sh, dt: torch.empty(sh, dtype=dt, device=dev)  # noqa: E731
+    a, b = empty(M, 0, dt=torch.uint8), empty(0, N, dt=torch.int8)
+    za = torch.full((M,), 7, dtype=torch.uint8, device=dev) if M > 1 else None
+    zb = torch.full((N,), -3, dtype=torch.int8, device=dev) if N > 1 else None
+    assert not olamd.matmul_integer(a, b).any()
+    assert not olamd.matmul_integer(a, b, za, zb).any()
+    s = [np.array(v, np.float32) for v in (0.02, 0.004, 0.3)]
+    for z in (0, 128):  # without and with column sums
+        q = olamd.qlinear_matmul(a, s[0], np.array(z, np.uint8), b, s[1], np.array(3, np.int8), s[2], np.array(9, np.uint8))
+        assert bool((q == 9).all())
+    for dt in (torch.float16, torch.bfloat16):
+        assert not olamd.matmul(empty(M, 0, dt=dt), empty(0, N, dt=dt)).any(), dt
+    scale = torch.full((N,), 0.5, device=dev) if N > 1 else torch.tensor(0.5, device=dev)
+    assert not olamd.dequantize_linear_matmul(empty(M, 0, dt=torch.float16), b, scale.half(), None, 1).any()
+    assert not olamd.dequantize_linear_matmul(empty(M, 0, dt=torch.bfloat16), b.view(torch.float8_e4m3fn), scale, None,
+                                              1, olamd.BFLOAT16).any()
