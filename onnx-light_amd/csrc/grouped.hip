@@ -198,6 +198,7 @@ namespace {
 // not know the groups' sizes: every group is taken a tenth larger than the
 // average, since a few rows past a multiple of r cost a whole tile row.
 int64_t GroupedRounds(const GroupedParams &p, int64_t r, int64_t c) {
+  if (p.G == 0) return 0;  // no group: no tile, and nothing to divide among
   const int64_t avg = (p.M * p.S + p.G - 1) / p.G, rows = avg + avg / 10;
   return mg::Rounds(p.G * ((rows + r - 1) / r) * ((p.N + c - 1) / c));
 }

@@ -59,6 +59,24 @@ def test_empty(olamd, dev, dt, M, S):
     assert tuple(y.shape) == (M, S, 32), n
 
 
+@pytest.mark.parametrize("K,N", [(64, 32), (50, 20), (0, 32)])
+def test_no_groups(olamd, dev, K, N):
+    """Weights [0, K, N]: every index lies outside, so every row is NaN."""
+    idx = torch.zeros((5, 2), dtype=torch.int64, device=dev)
+    for tdt in (torch.float16, torch.bfloat16):
+        for tb in (0, 1):
+            y = olamd.grouped_matmul(torch.ones((5, K), dtype=tdt, device=dev),
+                                     torch.ones((0, N, K) if tb else (0, K, N), dtype=tdt, device=dev), idx, None, tb,
+                                     check=False)
+            assert tuple(y.shape) == (5, 2, N) and bool(torch.isnan(y).all())
+    # quantized experts, on the fp8 and on the general path
+    for x, cast in ((torch.float8_e4m3fn, olamd.BFLOAT16), (torch.int8, olamd.BFLOAT16)):
+        y = olamd.dequantize_linear_grouped_matmul(torch.ones((5, K), dtype=torch.bfloat16, device=dev),
+                                                   torch.empty((0, K, N), dtype=x, device=dev),
+                                                   torch.tensor(0.5, device=dev), idx, cast_to=cast)
+        assert tuple(y.shape) == (5, 2, N) and bool(torch.isnan(y).all())
+
+
 SHAPES = [
     # M, K, N, G, S, transB, bias, index dtype
     (300, 256, 128, 8, 2, 0, False, np.int64),   # core, 3 routed tile-rows per group on average
