@@ -284,6 +284,34 @@ def test_qlinear_past_int32_signed_and_1d(olamd, oracle, dev, a_shape, b_shape):
     assert ref.reshape(-1)[0] == ref.min() < -100  # the sum past int32 is the most negative output
 
 
+@pytest.mark.parametrize("M,K,N", [(5, 256, 64), (24, 2048, 130), (70, 100, 33), (200, 64, 272), (1024, 64, 1088),
+                                   (2048, 64, 4096), (3, 140000, 24)], ids=str)
+@pytest.mark.parametrize("ydt", [np.int8, np.uint8])
+def test_qlinear_combined_scale_not_finite(olamd, oracle, dev, M, K, N, ydt):
+    """a_scale * b_scale / y_scale infinite: a zero sum makes a NaN, which the
+    reference's conversion turns into 0, and every other sum saturates.  NaN:
+    every result is 0.  Decode GEMM, small tiles, both tile heights of the
+    pipelined one, int64 sums."""
+    rng = np.random.default_rng(M + K + N)
+    a = rng.integers(0, 256, (M, K)).astype(np.uint8)
+    a[:: 2] = 77  # rows of zeros
+    b = rng.integers(-128, 128, (K, N)).astype(np.int8)
+    ta, tb = T(a, dev), T(b, dev)
+    acc = ((ta.double() - 77) @ (tb.double() - 5)).cpu().numpy()
+    info = np.iinfo(ydt)
+    for scales, want in (((100.0, 100.0, 1e-38), np.where(acc > 0, info.max, np.where(acc < 0, info.min, 0))),
+                         ((100.0, 100.0, -1e-38), np.where(acc < 0, info.max, np.where(acc > 0, info.min, 0))),
+                         ((np.nan, 1.0, 1.0), np.zeros_like(acc))):
+        s = [np.array(v, np.float32) for v in scales]
+        if M * K * N < 1_000_000:
+            with np.errstate(over="ignore", invalid="ignore"):
+                ref = oracle.qlinear_matmul(a, s[0], 77, b, s[1], 5, s[2], 9, y_dtype=olamd._torch_code(
+                    torch.int8 if ydt == np.int8 else torch.uint8))
+            assert np.array_equal(ref, want.astype(ydt))
+        y = olamd.qlinear_matmul(ta, s[0], np.array(77, np.uint8), tb, s[1], np.array(5, np.int8), s[2], np.array(9, ydt))
+        assert np.array_equal(y.cpu().numpy(), want.astype(ydt)), scales
+
+
 def test_qlinear_scalars_host_device_mixed(olamd, oracle, dev):
     """The six scalars read in one pass: device-resident ones copied on the
     call's stream with one synchronisation, host ones read directly; every
