@@ -89,3 +89,36 @@ def test_general_weights(olamd, dev, K, N, block, bf16):
             if bits == 4:
                 pw = olamd.prepare_weight(nibbles(w), code, (K, N))
                 assert torch.equal(olamd.dequantize_linear_matmul(a, pw, scale, zb, x_dtype=code, **kw), want)
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 40, 2000])
+@pytest.mark.parametrize("K,N", [(32, 48), (160, 80), (640, 272), (1696, 1040)], ids=str)
+@pytest.mark.parametrize("block", [8, 32, 0, -1])
+def test_padding_of_large_scales(olamd, dev, M, K, N, block):
+    """Rows past K, and whole groups past a wave's share, add nothing where a
+    padding code times the scale overflows fp16, or the scale is infinite: one-hot
+    rows of weights that stay below 65504, then ones times an infinite weight."""
+    g = torch.Generator(device=dev).manual_seed(M + K + N + block)
+    ints = lambda lo, hi, sh: torch.randint(lo, hi, sh, generator=g, device=dev, dtype=torch.int32)  # noqa: E731
+    shape, axis = ((K // block, N), 0) if block > 0 else (((N,), 1) if block == 0 else ((), 1))
+    full = lambda t: t.repeat_interleave(block, 0) if block > 0 else t  # noqa: E731
+    nibbles = lambda t: ((t.reshape(-1, 2)[:, 0] & 15) | (t.reshape(-1, 2)[:, 1] & 15) << 4).to(torch.uint8)  # noqa: E731
+    scale = torch.full(shape, 12000.0, dtype=torch.float16, device=dev)
+    at = ints(0, K, (M,)).long()
+    onehot = torch.zeros((M, K), dtype=torch.float16, device=dev)
+    onehot[torch.arange(M, device=dev), at] = 1
+    ones = torch.ones((M, K), dtype=torch.float16, device=dev)
+    for code, mid in ((olamd.INT4, 0), (olamd.UINT4, 8)):
+        w = ints(mid - 5, mid + 6, (K, N))
+        for zp in (mid != 0, True):
+            z = torch.full((max(2, scale.numel()),), mid, dtype=torch.int32, device=dev)
+            zb = (nibbles(z) if scale.numel() > 1 else nibbles(z)[:1]) if zp else None
+            pw = olamd.prepare_weight(nibbles(w), code, (K, N))
+            want = ((w - mid).float() * 12000.0).half()[at]
+            y = olamd.dequantize_linear_matmul(onehot, pw, scale, zb, axis=axis, x_dtype=code)
+            assert torch.equal(y, want), (code, zp)
+            inf = scale.clone()
+            inf[...] = float("inf")
+            up = olamd.prepare_weight(nibbles((w - mid).abs().clamp(1, 5) + mid), code, (K, N))
+            y = olamd.dequantize_linear_matmul(ones, up, inf, zb, axis=axis, x_dtype=code)
+            assert bool((y == float("inf")).all()), (code, zp)
