@@ -207,7 +207,9 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void TileGemmKernel(const 
 #pragma unroll
     for (int q = 0; q < NB; ++q) fb[d][q] = LoadPiece(pb[q] + tc * stepB);
   };
-  auto store = [&](const v4i(&a)[NA], const v4i(&b)[NB], char *st) __attribute__((always_inline)) {
+  // `left(q)`: bytes of B piece q that lie inside K (kSrcF8Chain: its padding
+  // becomes 0 after the scaling, which an infinite scale would make a NaN).
+  auto store = [&](const v4i(&a)[NA], const v4i(&b)[NB], char *st, auto left) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < NA; ++q) *reinterpret_cast<v4i *>(st + wa + 4096 * q) = a[q] ^ (int)aflip;
     char *sb = st + kASt;
@@ -224,6 +226,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void TileGemmKernel(const 
             const float *s = wsc[q] + 8 * h;
             w = v4i{(int)mg::PackBf16(f0.x * s[0], f0.y * s[1]), (int)mg::PackBf16(f1.x * s[2], f1.y * s[3]),
                     (int)mg::PackBf16(f2.x * s[4], f2.y * s[5]), (int)mg::PackBf16(f3.x * s[6], f3.y * s[7])};
+            if (left(q) == 0) w = v4i{0, 0, 0, 0};
           } else {
             w = v4i{mg::Fp8PairLo(x), mg::Fp8PairHi(x), mg::Fp8PairLo(y), mg::Fp8PairHi(y)};
           }
@@ -354,7 +357,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void TileGemmKernel(const 
 #pragma unroll
         for (int q = 0; q < NB; ++q) b[q] = TailBytes(Bb, b_total, pb[q] + t * stepB, nb[q], bflip);
       }
-      store(a, b, sm);
+      store(a, b, sm, [&](int q) { return nb[q]; });
       LdsBarrier();
       compute(sm);
       LdsBarrier();
@@ -364,7 +367,8 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void TileGemmKernel(const 
 #pragma unroll
     for (int d = 0; d < D; ++d) load(d, d);
     tail();
-    store(fa[0], fb[0], sg);
+    auto whole = [](int) { return 16; };
+    store(fa[0], fb[0], sg, whole);
     load(D, 0);
     LdsBarrier();
     for (int t = 0; t < rounds; t += D) {
@@ -372,7 +376,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void TileGemmKernel(const 
       for (int d = 0; d < D; ++d) {
         if (t + d >= rounds) break;
         const int n = (d + 1) % D;
-        store(fa[n], fb[n], sg + ((d + 1) & 1) * kStage);
+        store(fa[n], fb[n], sg + ((d + 1) & 1) * kStage, whole);
         load(t + d + 1 + D, n);
         if (G == 1 || t + d < steps) compute(sg + (d & 1) * kStage);
         LdsBarrier();

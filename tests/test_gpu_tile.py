@@ -176,3 +176,15 @@ def test_empty_k(olamd, dev, M, N):
     assert not olamd.dequantize_linear_matmul(empty(M, 0, dt=torch.float16), b, scale.half(), None, 1).any()
     assert not olamd.dequantize_linear_matmul(empty(M, 0, dt=torch.bfloat16), b.view(torch.float8_e4m3fn), scale, None,
                                               1, olamd.BFLOAT16).any()
+
+
+# fp8 weights with an infinite scale, K no multiple of a step: the padding of the
+# last step stays out of the sums.
+@pytest.mark.parametrize("M,K,N", [(5, 100, 40), (130, 100, 130), (3, 77, 17), (1100, 33, 2101), (40, 3073, 65)], ids=str)
+def test_fp8_infinite_scale(olamd, dev, M, K, N):
+    a = torch.ones((M, K), dtype=torch.bfloat16, device=dev)
+    w = torch.ones((K, N), device=dev).to(torch.float8_e4m3fn)
+    scale = torch.ones(N, device=dev)
+    scale[1] = float("inf")
+    y = olamd.dequantize_linear_matmul(a, w, scale, None, 1, olamd.BFLOAT16)
+    assert torch.equal(y, (scale * K).to(torch.bfloat16).expand(M, N))
