@@ -344,8 +344,6 @@ void LaunchHMatMul(const HMatMulParams &p, hipStream_t stream) {
 void LaunchHMatMulBT(const HMatMulParams &p, hipStream_t stream) {
   if (p.M == 0 || p.N == 0) return;
   const mg::GemmArgs g = HArgs(p);
-  if (p.N % 16 != 0 && p.M > 65535)
-    throw Unsupported("MatMul with B given as [N, K]: N % 16 != 0 takes at most 65535 rows");
   const bool core = mg::EligibleBT(g), small = tg::PrefersSmallTile(g, core);
   const bool half = mg::PrefersHalfTile<mg::kH16>(g);
   if (small || !core) LaunchHTileBT(g, p.bf16, !small, stream);

@@ -79,7 +79,7 @@ def test_16_bit(olamd, dev, shape):
     assert torch.equal(y, (exact[0] * scale.double()).to(torch.float32).to(torch.bfloat16))
 
 
-@pytest.mark.parametrize("M,N,K", [(9, 1, 64), (65, 63, 32), (130, 129, 320), (1100, 2101, 96)])
+@pytest.mark.parametrize("M,N,K", [(9, 1, 64), (65, 63, 32), (130, 129, 320), (1100, 2101, 96), (65537, 17, 32)])
 def test_b_transposed(olamd, dev, M, N, K):
     """The packed-weight product past the GEMVs: its decoded weight is [N, K]."""
     g = torch.Generator(device=dev).manual_seed(N)
