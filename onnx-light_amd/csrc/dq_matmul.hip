@@ -179,12 +179,22 @@ __global__ __launch_bounds__(256) void DequantRowsKernel(const DqMatMulParams p,
   }
 }
 
+// Weights of up to this many values give the vector kernels too few threads to
+// hide their longer chains: the value-per-thread kernel takes them.  With the
+// product, 32 rows, value per thread -> vector: uint8 256 x 512 with zero points 7.1 ->
+// 10.2 us, 512 x 1024 9.1 -> 11.5, 1024 x 1024 13.3 -> 14.3, 1024 x 2048 15.6 -> 15.6,
+// 2048 x 2048 26.2 -> 22.8; int4 tiled 512 x 512 8.4 -> 10.4, 1024 x 1024 13.7 -> 13.8,
+// 1024 x 2048 16.2 -> 14.9.  Pairs of columns make four times the threads of eights
+// (uint8 256 x 514 7.6 -> 8.4, 512 x 1026 10.0 -> 10.1, 1024 x 2050 18.4 -> 15.1).
+constexpr int64_t kSmallWeight = int64_t(1) << 20;
+
 void LaunchDequantWeight(const DqMatMulParams &p, uint16_t *out, hipStream_t stream) {
   const int64_t total = p.K * p.N, cols = (p.N + 63) / 64, ngroups = (p.K + 127) / 128;
   const bool k32 = p.K <= 0x7fffffff && p.block <= 0x7fffffff;
-  if (p.w_tiled && k32 && (p.mode != 2 || p.block % 8 == 0) && ngroups <= 65535 && cols <= 0x7fffffff) {
+  if (p.w_tiled && k32 && total > kSmallWeight && (p.mode != 2 || p.block % 8 == 0) && ngroups <= 65535 && cols <= 0x7fffffff) {
     hipLaunchKernelGGL(DequantTiledKernel, dim3((unsigned)cols, (unsigned)ngroups), dim3(256), 0, stream, p, out);
-  } else if (!p.w_tiled && k32 && p.N % 2 == 0 && total <= (int64_t(1) << 32)) {
+  } else if (!p.w_tiled && k32 && p.N % 2 == 0 && total > kSmallWeight / (p.N % 8 == 0 ? 1 : 4) &&
+             total <= (int64_t(1) << 32)) {
     const unsigned units = (unsigned)(total / (p.N % 8 == 0 ? 8 : 2)), per = 256 * kRowUnits;
     const dim3 grid((units + per - 1) / per);
     if (p.N % 8 == 0) hipLaunchKernelGGL(DequantRowsKernel<8>, grid, dim3(256), 0, stream, p, units, out);
@@ -310,7 +320,10 @@ void LaunchInt4Gemm(const DqMatMulParams &p, hipStream_t stream) {
 // A 4-bit weight in the ONNX packing past its GEMV's rows: tiled into scratch,
 // then as a prepared one.  Never more scratch than the dequantised weight of
 // the general path.  K = 4096, N = 11008: the pass takes 10 us (dequantising it 128),
-// 17 rows 125 -> 22.6 us, 1000 rows 204 -> 119.
+// 17 rows 125 -> 22.6 us, 1000 rows 204 -> 119.  A small weight whose last columns
+// or rows the pass would gather byte by byte is dequantised instead (32 rows,
+// dequantised -> tiled: 64 x 64 7.3 -> 11.2 us, 256 x 514 7.6 -> 11.5, 512 x 1026
+// 10.0 -> 12.0; 1024 x 2050 18.2 -> 12.9; whole ones 512 x 512 8.3 -> 7.4).
 DqMatMulParams WithTiledWeight(const DqMatMulParams &p, const void *scratch) {
   DqMatMulParams t = p;
   t.W = static_cast<const uint8_t *>(scratch);
@@ -320,7 +333,8 @@ DqMatMulParams WithTiledWeight(const DqMatMulParams &p, const void *scratch) {
 
 bool TilesFirst(const DqMatMulParams &p) {
   if (p.w_tiled || (p.w_dtype != kInt4 && p.w_dtype != kUint4) || p.K == 0 || p.N % 2 != 0 ||
-      TiledInt4Bytes(p.K, p.N) > p.K * p.N * 2)
+      TiledInt4Bytes(p.K, p.N) > p.K * p.N * 2 ||
+      (p.K * p.N <= kSmallWeight && (p.N % 8 != 0 || p.K % 128 != 0)))
     return false;
   const DqMatMulParams t = WithTiledWeight(p, reinterpret_cast<const void *>(uintptr_t(256)));
   return GemvQ4TiledEligible(t) || Int4GemmEligible(t);
