@@ -64,6 +64,7 @@ template <int OUT, bool CV = false> void LaunchIGemmFastOut(const IGemmParams &p
 }
 
 void LaunchIGemmFastI32(const IGemmParams &p, bool half, hipStream_t s);
+void LaunchIGemmFastDev(const IGemmParams &p, bool half, hipStream_t s);
 void LaunchIGemmFastQ8(const IGemmParams &p, bool half, hipStream_t s);
 void LaunchIGemmFastQ8Row(const IGemmParams &p, bool half, hipStream_t s);
 void LaunchIGemmConvI32(const IGemmParams &p, bool half, hipStream_t s);

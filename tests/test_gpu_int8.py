@@ -312,6 +312,24 @@ def test_qlinear_combined_scale_not_finite(olamd, oracle, dev, M, K, N, ydt):
         assert np.array_equal(y.cpu().numpy(), want.astype(ydt)), scales
 
 
+@pytest.mark.parametrize("M,K,N", [(1024, 1088, 1088), (2048, 1024, 4096)], ids=str)
+def test_device_zero_points_on_the_pipelined_kernel(olamd, dev, M, K, N):
+    """Single zero points in device memory, both tile heights: neutral ones (the
+    K loop without row and column sums), one of the two, a missing one, others."""
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    for adt in (torch.uint8, torch.int8):
+        for bdt in (torch.uint8, torch.int8):
+            ints = lambda sh, dt: torch.randint(-128, 128, sh, generator=g, device=dev, dtype=torch.int32)  # noqa: E731
+            a, b = (ints((M, K), adt) + (128 if adt == torch.uint8 else 0)).to(adt), \
+                   (ints((K, N), bdt) + (128 if bdt == torch.uint8 else 0)).to(bdt)
+            na, nb = (128 if adt == torch.uint8 else 0), (128 if bdt == torch.uint8 else 0)
+            for za, zb in ((na, nb), (na, nb + 5), (na + 3, nb), (na - 7, nb + 2), (na, None), (None, nb)):
+                ta = None if za is None else torch.tensor(za, dtype=adt, device=dev)
+                tb = None if zb is None else torch.tensor([zb], dtype=bdt, device=dev)
+                want = (a.double() - (za or 0)) @ (b.double() - (zb or 0))
+                assert torch.equal(olamd.matmul_integer(a, b, ta, tb).double(), want), (za, zb)
+
+
 def test_qlinear_scalars_host_device_mixed(olamd, oracle, dev):
     """The six scalars read in one pass: device-resident ones copied on the
     call's stream with one synchronisation, host ones read directly; every
