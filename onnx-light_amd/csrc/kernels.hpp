@@ -70,8 +70,7 @@ __device__ inline float DevScale(const void *p, int f16) {
   return f16 ? (float)*static_cast<const _Float16 *>(p) : *static_cast<const float *>(p);
 }
 
-// Host values (alpha, beta, cs, zy) overridden by the device-resident ones;
-// cs comes out finite.
+// Host values (alpha, beta, cs, zy) overridden by the device-resident ones.
 __device__ inline QResolved ResolveQ(const QDevScalars &d, int a_u8, int b_u8, int y_signed, int32_t alpha,
                                      int32_t beta, float cs, float zy) {
   QResolved r{alpha, beta, cs, zy};
@@ -85,11 +84,14 @@ __device__ inline QResolved ResolveQ(const QDevScalars &d, int a_u8, int b_u8, i
     r.cs = ab / sy;
   }
   if (d.zy) r.zy = (float)(y_signed ? (int32_t)(int8_t)d.zy[0] : (int32_t)d.zy[0]);
-  // A combined scale that is not finite, replaced once by constants whose
-  // clamped results are the same, so that no epilogue looks for a NaN per
-  // value: infinite times a zero sum, and anything times a NaN, land as 0
-  // whatever the zero point (the x86-64 conversion of a NaN); every other sum
-  // saturates.
+  return r;
+}
+
+// A combined scale that is not finite, replaced once by constants whose clamped
+// results are the same, so that no epilogue looks for a NaN per value: infinite
+// times a zero sum, and anything times a NaN, land as 0 whatever the zero point
+// (the x86-64 conversion of a NaN); every other sum saturates.
+__device__ inline QResolved FiniteScale(QResolved r) {
   if (!(__builtin_fabsf(r.cs) < __builtin_huge_valf())) {
     r.cs = r.cs != r.cs ? 0.f : __builtin_copysignf(0x1p100f, r.cs);
     r.zy = 0.f;

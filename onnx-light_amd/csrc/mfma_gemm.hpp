@@ -894,6 +894,7 @@ __global__ __launch_bounds__(kThreads, MB == 2 && (KIND == kBf16F8 || KIND == kF
   // they are device-resident
   QResolved qv{p.alpha_scalar, p.beta_scalar, p.cs, p.zy};
   if constexpr (KIND == kI8) qv = ResolveQ(p.dev, p.a_u8, p.b_u8, p.y_signed, p.alpha_scalar, p.beta_scalar, p.cs, p.zy);
+  if constexpr (OUT == kOutQ8) qv = FiniteScale(qv);
   int32_t *zc = zsum + (KIND == kI8 && ZP ? wave * 2 * kWN : 0);
   int zrow[MB] = {};
   if constexpr (KIND == kI8 && ZP) {

@@ -273,6 +273,7 @@ __global__ __launch_bounds__(64 * W, CW == 8 && MT == 2 ? 2 : 4) void SkinnyKern
     }
     QResolved qv{p.alpha_scalar, p.beta_scalar, p.cs, p.zy};
     if constexpr (I8) qv = ResolveQ(p.dev, p.a_u8, p.b_u8, p.y_signed, p.alpha_scalar, p.beta_scalar, p.cs, p.zy);
+    if constexpr (OUT == mg::kOutQ8) qv = FiniteScale(qv);
     const int mone = tr / 16;  // ZP: the operand that holds the row of ones (tr < 16 MT)
 #pragma unroll
     for (int m = MT - 1; m >= 0; --m) {

@@ -408,6 +408,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void TileGemmKernel(const 
   // ---- zero-point terms (mod 2^32): Y = sum a'b' + beta_j RA_i + alpha_i Q_j, Q_j = CB_j + K beta_j ----
   QResolved qv{p.alpha_scalar, p.beta_scalar, p.cs, p.zy};
   if constexpr (I8) qv = ResolveQ(p.dev, p.a_u8, p.b_u8, p.y_signed, p.alpha_scalar, p.beta_scalar, p.cs, p.zy);
+  if constexpr (OUT == mg::kOutQ8) qv = FiniteScale(qv);
   int32_t *zc = zsum + (ZP ? wave * 2 * kWN : 0);
   if constexpr (ZP) {
 #pragma unroll
