@@ -62,8 +62,8 @@ def test_fp8(olamd, dev, M, K, N):
     assert torch.equal(y, (a.double() @ w.double() * scale.double()).to(torch.float32).to(torch.bfloat16))
 
 
-@pytest.mark.parametrize("M,G,K,N", [(1, 3, 64, 64), (40, 4, 288, 112), (64, 16, 256, 1040), (90, 3, 1024, 4112)],
-                         ids=str)
+@pytest.mark.parametrize("M,G,K,N", [(1, 3, 64, 64), (40, 4, 288, 112), (64, 16, 256, 1040), (90, 3, 1024, 4112),
+                                     (260, 200, 64, 80), (5, 4096, 32, 64)], ids=str)
 def test_grouped(olamd, dev, M, G, K, N):
     g = torch.Generator(device=dev).manual_seed(M + N)
     a, w = _ints(g, -2, 3, (M, K)), _ints(g, -4, 5, (G, K, N))
@@ -82,3 +82,12 @@ def test_grouped(olamd, dev, M, G, K, N):
                 continue
             r = (a[m].double() @ w[e].double() * scale[e, 0].double()).to(torch.float32).to(torch.bfloat16)
             assert torch.equal(y[m, s], (r.float() + bias[e].float()).to(torch.bfloat16)), (m, s)
+
+
+def test_grouped_none_inside(olamd, dev):
+    a = torch.ones((9, 64), dtype=torch.bfloat16, device=dev)
+    w = torch.ones((5, 64, 144), device=dev).to(torch.float8_e4m3fn)
+    for bad in (-1, 5):
+        y = olamd.dequantize_linear_grouped_matmul(a, w, torch.ones((5, 1, 144), device=dev),
+                                                   torch.full((9, 2), bad, device=dev), cast_to=olamd.BFLOAT16)
+        assert bool(torch.isnan(y).all())
