@@ -203,6 +203,26 @@ int64_t GroupedRounds(const GroupedParams &p, int64_t r, int64_t c) {
   return mg::Rounds(p.G * ((rows + r - 1) / r) * ((p.N + c - 1) / c));
 }
 
+// Whether 16-bit groups take 128-row tiles, whose round of the chip takes about
+// 0.6 of a 256-row one's: where no routing, or hardly any, makes more rounds of
+// them.  The host does not know the groups' sizes.
+//  - At most one round of them however the pairs fall (top-2, 64 tokens, 4 experts
+//    [4096, 4096]: even 44.7 -> 33.8 us, all to one 45.0 -> 30.0).
+//  - Up to 128 pairs: as many tiles of either height (64 tokens, 8 experts [14336,
+//    4096]: even 172 -> 160, all to one 122 -> 76).
+//  - Up to 256: one more row of tiles at most, which costs a round only where the
+//    256-row tiles fill just one (128 tokens, 8 experts [4096, 14336]: even 203 ->
+//    193, skewed 220 -> 183).
+// Past that the better height depends on the routing: 256-row -> 128-row tiles, 8
+// experts [4096, 14336]: 2048 tokens, even 563 -> 717 us, all to one 414 -> 521; 256
+// tokens, even 220 -> 197, all to one 59 -> 70; [14336, 4096], 128 tokens, skewed 175
+// -> 249.
+bool PrefersHalfGroups(const GroupedParams &p) {
+  const int64_t P = p.M * p.S, most = std::min(P, p.G);  // groups with any pair
+  if ((P + 127 * most) / 128 * p.nbn <= 256 || P <= 128) return true;
+  return P <= 256 && most * p.nbn > 512;
+}
+
 template <int OUT, int GM> void LaunchGroupedCore(const mg::GemmArgs &g, int64_t tiles, bool half, hipStream_t s) {
   if (half) mg::LaunchGrouped<OUT, GM, mg::kH16, 2, 2>(g, tiles, s);
   else mg::LaunchGrouped<OUT, GM>(g, tiles, s);
@@ -214,10 +234,7 @@ void LaunchGroupedMatMul(const GroupedParams &gp, hipStream_t stream) {
   GroupedParams p = gp;
   const int64_t P = p.M * p.S;
   if (P == 0 || p.N == 0) return;
-  // 128-row tiles where they take less than 20 / 12 of the 256-row ones' rounds
-  // (as PrefersHalfTile; bf16, 4 experts [4096, 4096] given [N, K], top-2: 256
-  // tokens 46.5 -> 36.6 us, 500 tokens 51.2 against 62.5 us)
-  const bool half = 12 * GroupedRounds(p, 128, 128) < 20 * GroupedRounds(p, 256, 128);
+  const bool half = PrefersHalfGroups(p);
   p.tile_rows = half ? 128 : 256;
   hipLaunchKernelGGL(GroupRouteKernel, dim3(1), dim3(kRouteThreads), GroupedRouteLds(p.G), stream, p);
   if (p.K == 0 || !GroupedCoreEligible(p)) {

@@ -188,3 +188,21 @@ def test_fp8_infinite_scale(olamd, dev, M, K, N):
     scale[1] = float("inf")
     y = olamd.dequantize_linear_matmul(a, w, scale, None, 1, olamd.BFLOAT16)
     assert torch.equal(y, (scale * K).to(torch.bfloat16).expand(M, N))
+
+
+# 16-bit groups in 128-row tiles (few pairs, or few tiles) and in 256-row ones, even
+# and skewed.
+@pytest.mark.parametrize("M,G,K,N", [(50, 8, 96, 2064), (100, 8, 64, 9008), (100, 8, 64, 6016), (300, 8, 64, 6016),
+                                     (600, 3, 160, 1040)], ids=str)
+def test_grouped_tile_heights(olamd, dev, M, G, K, N):
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    ints = lambda lo, hi, sh: torch.randint(lo, hi, sh, generator=g, device=dev, dtype=torch.int32)  # noqa: E731
+    a, w = ints(-2, 3, (M, K)), ints(-4, 5, (G, K, N))
+    for idx in (ints(0, G, (M, 2)), (torch.rand((M, 2), generator=g, device=dev) ** 4 * G).int().clamp(0, G - 1)):
+        every = torch.stack([a.double() @ w[e].double() for e in range(G)])  # [G, M, N]
+        want = torch.stack([every[idx[:, s].long(), torch.arange(M, device=dev)] for s in range(2)], dim=1).float()
+        for dt in (torch.float16, torch.bfloat16):
+            y = olamd.grouped_matmul(a.to(dt), w.to(dt), idx, transB=0)
+            assert torch.equal(y, want.to(dt)), dt
+            y = olamd.grouped_matmul(a.to(dt), w.transpose(1, 2).contiguous().to(dt), idx, transB=1)
+            assert torch.equal(y, want.to(dt)), dt
