@@ -325,8 +325,11 @@ int onnxl_amd_dequantize_linear_matmul(const onnxl_amd_tensor *a, const onnxl_am
  * - its scratch is a fixed array of 8 MiB per device, held until the process
  *   ends: 64 KiB of counters (16384, one per 256-column strip of the ONNX-
  *   layout int4 GEMV) and 8128 KiB for split-K partial sums or a dequantised
- *   weight.  A call that needs more returns ONNXL_AMD_UNSUPPORTED, naming the
- *   sizes (the allocating entry point then serves it);
+ *   weight.  A call that counts as more returns ONNXL_AMD_UNSUPPORTED, naming the
+ *   sizes (the allocating entry point then serves it).  GEMV calls count as
+ *   their scratch, fp8 weights of the pipelined GEMM's shapes as none, all
+ *   others as their weight dequantised to 16 bits, also where the kernel that
+ *   takes them needs less;
  * - it calls no hipMalloc / hipFree.
  * All calls on one device share that array: calls that overlap on one device
  * (different streams, or different threads without ordering) race.  The

@@ -1565,8 +1565,8 @@ int DqMatMulNoAlloc(const onnxl_amd_tensor *a, const onnxl_amd_tensor *x, const 
   p.Y = y->data;
   const size_t need = DqMatMulFixedScratchBytes(p), nc = DqMatMulCounters(p);
   if (need > kNoAllocDataBytes || nc * sizeof(unsigned) > kNoAllocCounterBytes)
-    throw Unsupported(Cat(kDqmName, ": this call needs ", need, " bytes of scratch and ", nc,
-                          " counters; the no-allocation entry point holds ", kNoAllocDataBytes, " bytes and ",
+    throw Unsupported(Cat(kDqmName, ": this call counts as ", need, " bytes (its scratch, or its dequantised weight) and ",
+                          nc, " counters; the no-allocation entry point holds ", kNoAllocDataBytes, " bytes and ",
                           kNoAllocCounterBytes / sizeof(unsigned), " counters (use the allocating entry point)"));
   if (!LaunchDqMatMul(p, base + kNoAllocCounterBytes, kNoAllocDataBytes, reinterpret_cast<unsigned *>(base),
                       kNoAllocCounterBytes / sizeof(unsigned), stream))

@@ -374,9 +374,12 @@ size_t DqMatMulScratchBytes(const DqMatMulParams &p) {
   return (size_t)(p.K * p.N) * sizeof(uint16_t);
 }
 
-// The scratch that bounds the no-allocation entry point: a call whose weight
-// would not fit there dequantised is refused, also where the kernel that
-// takes it needs none.
+// The bytes that the no-allocation entry point counts a call with, against its
+// fixed array: the scratch of the GEMVs, none for an fp8 weight of the pipelined
+// GEMM's shapes, and for every other call its dequantised weight, whatever kernel
+// takes it.  So the calls it accepts depend on sizes and types alone: a line between
+// two kernels that moves (PrefersGemv, TilesFirst) turns no captured call away.
+// Never less than DqMatMulScratchBytes.
 size_t DqMatMulFixedScratchBytes(const DqMatMulParams &p) {
   if (p.M <= 16 && GemvQ4TiledEligible(p)) return 0;
   if (GemvQ4Eligible(p)) return GemvQ4ScratchBytes(p);

@@ -206,3 +206,16 @@ def test_grouped_tile_heights(olamd, dev, M, G, K, N):
             assert torch.equal(y, want.to(dt)), dt
             y = olamd.grouped_matmul(a.to(dt), w.transpose(1, 2).contiguous().to(dt), idx, transB=1)
             assert torch.equal(y, want.to(dt)), dt
+
+
+# A weight past 2^31 bytes, N odd: one-hot rows pick rows of it, its last among them.
+@pytest.mark.parametrize("M", [8, 40])  # the decode GEMM, tiles
+def test_weight_past_two_gib(olamd, dev, M):
+    K, N = 32800, 65537
+    b = torch.empty((K, N), dtype=torch.int8, device=dev)
+    for k in range(0, K, 4100):
+        b[k:k + 4100] = torch.randint(-128, 128, (4100, N), device=dev, dtype=torch.int8)
+    at = torch.linspace(0, K - 1, M, device=dev).long()
+    a = torch.zeros((M, K), dtype=torch.int8, device=dev)
+    a[torch.arange(M, device=dev), at] = 3
+    assert torch.equal(olamd.matmul_integer(a, b), b[at].int() * 3)

@@ -72,6 +72,14 @@ def test_noalloc_rejections(olamd, oracle, dev):
     s = torch.ones((N,), dtype=torch.float16, device=dev)
     with pytest.raises(olamd.Unsupported, match="no-allocation entry point holds"):
         olamd.dequantize_linear_matmul_noalloc(a, x, s, None, axis=1)
+    # a prepared 4-bit weight past the GEMV's 16 rows counts as dequantised too, at any
+    # row count, also where the kernel that takes it needs no scratch
+    pw = olamd.prepare_weight(torch.zeros((K * N // 2,), dtype=torch.uint8, device=dev), olamd.INT4, (K, N))
+    for rows in (17, 64, 500):
+        with pytest.raises(olamd.Unsupported, match="no-allocation entry point holds"):
+            olamd.dequantize_linear_matmul_noalloc(torch.zeros((rows, K), dtype=torch.float16, device=dev), pw, s, None,
+                                                   axis=1, x_dtype=olamd.INT4)
+    olamd.dequantize_linear_matmul_noalloc(a[:16], pw, s, None, axis=1, x_dtype=olamd.INT4)
     # host payloads are refused (no staging without allocation)
     a_h, x_h, s_h, _ = _int4_case(oracle, rng, 2, 256, 64, 32, False, torch.device("cpu"))
     with pytest.raises(olamd.InvalidArgument, match="device payloads only"):
