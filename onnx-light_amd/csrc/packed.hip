@@ -1480,13 +1480,16 @@ __global__ __launch_bounds__(256) void GemvKLdsKernel(const uint16_t *__restrict
 }
 
 // q4_k, up to kQ4kRows activation rows: 16 code bytes per lane (8 lanes per
-// block), both nibbles of each, so a lane decodes two scales for 32 values.  The
-// staged kernel is bound by its VALU work: 8 values per lane cost a whole scale
-// decode, and each code an extract and a conversion of its own.  Here a masked
+// block), both nibbles of each, so a lane decodes two scales for 32 values.  In
+// the staged kernel 8 values per lane cost a whole scale decode, and each code an
+// extract and a conversion of its own (1608 VALU instructions per wave at
+// [14336, 4096], M = 1, against 958 here).  Here a masked
 // dword is a pair of codes as fp16 denormals (q * 2^-24; the high nibbles
 // q * 2^-20), which the mixed-precision multiply-add takes as it is, its fp32
 // scale carrying the power of two: exact, so the rounding stays that of DecodeK.
-// Per 8 values 5 extracts, 8 multiply-adds and 4 dot products; those bound it.
+// Per 8 values 5 extracts, 8 multiply-adds and 4 dot products.  No unit is full:
+// VALU issue 47% of the SIMDs' cycles, 2.4 TB/s; a wave's two steps there are its
+// first load's latency, then a dependent decode.
 // The header's dwords go to the lanes of a quad, one each, and round by DPP.
 constexpr int kQ4kRows = 4;
 // Where most of a wave's 8 blocks per step are there.  Staged kernel against this

@@ -455,10 +455,13 @@ inline bool PrefersSkinny(const mg::GemmArgs &p, bool i8, bool zp) {
 
 // Whether a grouped call goes here instead of the routed core, whose tiles are
 // nearly empty then: by the average number of pairs per expert and the columns
-// of all experts.  bf16 x fp8 experts, K = 4096, here against the core's 128-row
-// tiles: 8 x N = 14336 with 8 / 16 / 32 pairs per expert 101 / 117 / 178 against
-// 107 / 114 / 120 us; 8 x N = 4096 with 16 / 32 pairs 25.8 / 41.5 against 33.1 / 33.8
-// us; 8 x N = 1024 with 32 / 64 pairs 29.8 / 46.4 against 31.5 / 32.7 us.
+// of all experts.  bf16 x fp8 experts, K = 4096, evenly routed, here against the
+// core's 128-row tiles: 8 x N = 14336 with 8 / 12 / 16 / 32 pairs per expert 100 / 109 /
+// 117 / 164 against 107 / 109 / 110 / 115 us; 8 x N = 4096 with 16 / 32 pairs 26.6 / 49.3
+// against 34.1 / 38.2; 8 x N = 1024 with 32 / 64 / 128 pairs 21.1 / 22.6 / 41.4 against
+// 30.9 / 31.6 / 31.8 (the line is below what 64 would allow).  Skewed routing, where
+// busy experts' columns are read once per 16 pairs: 8 x 14336 with 12 pairs 122 against 113,
+// 8 x 4096 with 16 pairs 41.4 against 34.6.
 inline bool PrefersSkinnyGrouped(const mg::GemmArgs &p) {
   const int64_t pairs = p.M * p.grp_sel, cols = p.grp_count * p.N;
   const int64_t most = cols <= 16384 ? 32 : (cols <= 65536 ? 16 : 12);

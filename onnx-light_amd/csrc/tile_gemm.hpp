@@ -550,17 +550,17 @@ inline int64_t Tiles(const GemmArgs &p, int side) {
 // to one of them per CU: at K = 4096, int8 / fp8 / fp16, 256 x 4096 outputs (256
 // small tiles) take 14.1 / 24.0 / 23.7 us here and 15.5 / 25.6 / 24.2 us in the
 // core's 128 x 128 tiles; 512 x 4096 (512 small tiles) 21.4 / 35.4 / 34.3 against
-// 16.7 / 26.6 / 25.6 us, the small tile's LDS traffic per product being twice the
-// core's.  The shapes the core does not take go on to two per CU, then to
+// 16.7 / 26.6 / 25.6 us: a small tile reads each operand byte for half as many
+// products as the core's.  The shapes the core does not take go on to two per CU, then to
 // 128 x 128 tiles of this kernel (1024 x 4096: 39.4 -> 30.0 us int8, 67.1 -> 51.0 us
 // fp16; at 688 small tiles the two tie).
 inline bool PrefersSmallTile(const GemmArgs &p, bool core) { return Tiles(p, 64) <= (core ? 256 : 512); }
 
 // Whether the 64 x 64 tile takes two groups of waves per workgroup, each half of
 // the K steps: with at most one tile per CU, one group's step is a chain of LDS
-// writes, a barrier, LDS reads and four dependent MFMAs; two groups fill its
-// waits until the LDS itself is the bound (32 KB read and 16 KB written per
-// step).  The exchange at the end costs about 1 us, so it pays for long K: fp16,
+// writes, a barrier, LDS reads and four dependent MFMAs; two groups fill part of
+// its waits (fp16 150 x 4096 x 4096 with two: the waves still wait half of their
+// time, the LDS is 30% and the matrix cores are 14% busy).  The exchange at the end costs about 1 us, so it pays for long K: fp16,
 // one -> two groups, 150 x 4096 outputs at K = 1536 9.5 -> 9.6 us, 2048 11.2 ->
 // 11.2, 3072 16.1 -> 15.3, 4096 22.6 -> 19.4, 8192 40.8 -> 32.9; fp8, whose
 // decode lengthens the chain, 1536 10.4 -> 9.9, 4096 21.4 -> 18.5 us.  int8
@@ -575,8 +575,10 @@ template <int KIND, int SRC> inline bool PrefersTwoGroups(const GemmArgs &p) {
 }
 
 // Whether 64 x 128 tiles take a problem of more 64 x 64 tiles than CUs: at most
-// one per CU, they keep any CU from two of the small ones, whose LDS traffic (48
-// KB a step, against 72 for twice the outputs) does not overlap.  335 x 3001
+// one per CU, they keep any CU from two of the small ones: twice the outputs for
+// one chain of steps and half again the LDS traffic (72 KB a step against 48).
+// Neither unit is near full then (u8 335 x 3001, K = 1001: LDS 7%, matrix cores 4%,
+// 0.6 waves per SIMD): the chain's latency bounds it.  335 x 3001
 // outputs, 64 x 64 -> 64 x 128: int8 K = 513 11.2 -> 8.8 us, 1001 13.0 -> 10.4, 4090
 // 29.3 -> 25.2; fp16 11.3 -> 10.2, 15.3 -> 13.1, 42.5 -> 35.2.  Steps in flight: two
 // for int8 (four: 9.9, 11.5, 25.0), four for fp16 (two: 9.7, 12.7, 39.2).  fp8 weights
