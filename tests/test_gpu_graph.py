@@ -141,17 +141,18 @@ def _qlm_scalars(rng, a, b, adt, bdt, ydt, a_s):
     return [np.array(a_s), np.array(za, adt), np.array(b_s), np.array(zb, bdt), np.array(y_s), np.array(zy, ydt)]
 
 
-# shapes reaching each int8 kernel: the pipelined MFMA core (K % 64 == 0,
-# N % 16 == 0), the byte-granular tail kernel (K = 200), the K-tail kernel
-# (N % 16 != 0) with a batch, and the int64-exact kernel (K = 45000 with
-# unread zero points counts as past the int32-exact bound)
+# operands of each kind: whole K steps and 16-byte rows, on the small tile (96
+# tiles of 64 x 64) and on the pipelined MFMA core (288), rows of 8 bytes
+# (K = 200), a row-major B off 16 bytes with a batch, and the int64-exact kernel
+# (K = 45000 with unread zero points counts as past the int32-exact bound)
 QLM_CAPTURE = [((512, 1024), (1024, 768), np.uint8, np.int8, np.uint8),
                ((300, 200), (200, 136), np.int8, np.int8, np.int8),
                ((3, 50, 128), (3, 128, 40), np.uint8, np.uint8, np.int8),
-               ((6, 45000), (45000, 40), np.int8, np.uint8, np.uint8)]
+               ((6, 45000), (45000, 40), np.int8, np.uint8, np.uint8),
+               ((1024, 128), (128, 1104), np.uint8, np.int8, np.uint8)]
 
 
-@pytest.mark.parametrize("a_shape,b_shape,adt,bdt,ydt", QLM_CAPTURE, ids=["core", "bytes", "ktail", "int64"])
+@pytest.mark.parametrize("a_shape,b_shape,adt,bdt,ydt", QLM_CAPTURE, ids=["core", "bytes", "ktail", "int64", "pipelined"])
 def test_qlinear_graph_device_scalars(olamd, oracle, dev, a_shape, b_shape, adt, bdt, ydt):
     """QLinearMatMul captured with its scalars in device memory (a_scale on the
     host): the kernels read them at replay time, so rewriting them between
@@ -196,8 +197,9 @@ def test_qlinear_graph_device_scalars(olamd, oracle, dev, a_shape, b_shape, adt,
 
 
 @pytest.mark.parametrize("a_shape,b_shape,adt,bdt", [((512, 1024), (1024, 512), np.uint8, np.int8),
-                                                     ((300, 200), (200, 136), np.int8, np.uint8)],
-                         ids=["core", "bytes"])
+                                                     ((300, 200), (200, 136), np.int8, np.uint8),
+                                                     ((1024, 1024), (1024, 1104), np.uint8, np.int8)],
+                         ids=["core", "bytes", "pipelined"])
 def test_matmul_integer_graph_device_zero_points(olamd, oracle, dev, a_shape, b_shape, adt, bdt):
     """MatMulInteger captured with one-element zero points in device memory:
     rewritten between replays (including to the values that make the row /
