@@ -214,10 +214,11 @@ def test_cast_vs_oracle(olamd, oracle, dev):
 # FLOAT16 / BFLOAT16 MatMul
 
 MM_SHAPES = [
-    ((300, 192), (192, 144)),        # MFMA core: tails in M and N
-    ((2, 64, 128), (128, 64)),       # MFMA core, batched A
+    ((300, 192), (192, 144)),        # small tiles: tails in M and N
+    ((2, 64, 128), (128, 64)),       # batched A
+    ((5, 320, 96), (5, 96, 784)),    # pipelined kernel (325 tiles of 64 x 64), batch, tails
     ((3, 1, 40, 64), (5, 64, 32)),   # broadcast batch dims
-    ((37, 45), (45, 29)),            # simple kernel (K % 64, N % 16)
+    ((37, 45), (45, 29)),            # rows off 16 bytes
     ((64,), (64, 40)),               # 1-D A
     ((8, 0), (0, 16)),               # K = 0
 ]
